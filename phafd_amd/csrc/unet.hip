@@ -487,17 +487,72 @@ __global__ __launch_bounds__(256) void k_conv_dw(const uint16_t *__restrict__ X,
       }
 }
 
-// G_w[co][ci][tap] += sum over the nb*4 partials (fixed order)
-__global__ void k_dw_reduce(const float *__restrict__ part, int nparts, int cin, int cout, int taps,
-                            float *__restrict__ gw) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int total = cin * cout * taps;
-  if (i >= total) return;
-  const int co = i % cout, ci = (i / cout) % cin, tap = i / (cout * cin);
-  const float *p = part + (size_t)tap * nparts * (cin * cout) + ci * cout + co;
+// The partials of one parameter gradient: part[tap][k][ci][co], k < nparts,
+// added up in ascending k and then to g[(co * cin + ci) * taps + tap] (a bias
+// or the head: one tap, one input channel).
+struct RedJob {
+  const float *part;
+  float *g;
+  int nparts, cin, cout, taps, first;   // first: the job's first block
+};
+constexpr int RED_JOBS = 20;
+struct RedJobs {
+  RedJob j[RED_JOBS];
+  int n, blocks;
+};
+constexpr int RED_ROWS = 128;   // partials staged at a time: 32 KB, four blocks per CU
+// Every gradient tensor's partials in one launch at the end of a backward
+// pass.  Up to 1024 partials of an output are added in one chain, in order
+// (the sums, and so a trained network, are those of a plain loop).  What
+// bounds such a loop is not the chain, 1024 adds of a few cycles, but a
+// memory latency per add: 64 outputs' partials therefore come to LDS a block
+// of rows at a time by all four waves (256 contiguous bytes a row), the next
+// rows in flight in registers while one wave adds the current ones.  At 64^3:
+// 71 us for the seventeen tensors (175 MB of partials), against 165 us per
+// bias, 143 us per weight tensor and 74 us for the head with a launch and a
+// loop over global memory each (84% of a training step).
+__global__ __launch_bounds__(256) void k_part_reduce(RedJobs jobs) {
+  __shared__ float buf[RED_ROWS][64];
+  int q = 0;
+  while (q + 1 < jobs.n && (int)blockIdx.x >= jobs.j[q + 1].first) q++;
+  const RedJob J = jobs.j[q];
+  const int per = J.cin * J.cout, total = per * J.taps;
+  const int c = threadIdx.x & 63, sl = threadIdx.x >> 6;
+  const int i = ((int)blockIdx.x - J.first) * 64 + c;
+  const bool on = i < total;
+  const int tap = on ? i / per : 0, r = on ? i - tap * per : 0;
+  const float *p = J.part + (size_t)tap * J.nparts * per + r;
+  constexpr int NR = RED_ROWS / 4;
+  float v[NR];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < NR; u++) {
+      const int k = k0 + sl + 4 * u;
+      v[u] = on && k < J.nparts ? p[(size_t)k * per] : 0.f;
+    }
+  };
   float s = 0.f;
-  for (int k = 0; k < nparts; k++) s += p[(size_t)k * cin * cout];
-  gw[((size_t)co * cin + ci) * taps + tap] += s;
+  fetch(0);
+  for (int k0 = 0; k0 < J.nparts; k0 += RED_ROWS) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NR; u++) buf[sl + 4 * u][c] = v[u];
+    __syncthreads();
+    if (k0 + RED_ROWS < J.nparts) fetch(k0 + RED_ROWS);
+    if (sl == 0) {
+      const int m = J.nparts - k0 < RED_ROWS ? J.nparts - k0 : RED_ROWS;
+      if (m == RED_ROWS) {
+#pragma unroll 16
+        for (int k = 0; k < RED_ROWS; k++) s += buf[k][c];
+      } else {
+        for (int k = 0; k < m; k++) s += buf[k][c];
+      }
+    }
+  }
+  if (sl == 0 && on) {
+    const int co = i % J.cout, ci = (i / J.cout) % J.cin;
+    J.g[((size_t)co * J.cin + ci) * J.taps + tap] += s;
+  }
 }
 
 // column sums of D[N][C] per block: part[blk][C]
@@ -515,13 +570,6 @@ __global__ __launch_bounds__(256) void k_colsum(const uint16_t *__restrict__ D, 
     for (int k = 0; k < PER; k++) t += red[k * C + threadIdx.x];
     part[(size_t)blockIdx.x * C + threadIdx.x] = t;
   }
-}
-__global__ void k_colsum_reduce(const float *__restrict__ part, int nb, int C, float *__restrict__ g) {
-  const int c = threadIdx.x;
-  if (c >= C) return;
-  float s = 0.f;
-  for (int k = 0; k < nb; k++) s += part[(size_t)k * C + c];
-  g[c] += s;
 }
 
 // ----------------------------------------------------- pooling / upsampling
@@ -659,14 +707,6 @@ __global__ __launch_bounds__(256) void k_head_bwd(const uint16_t *__restrict__ A
     part[(size_t)blockIdx.x * 17 + threadIdx.x] = t;
   }
 }
-__global__ void k_head_reduce(const float *__restrict__ part, int nb, float *__restrict__ gw, float *__restrict__ gb) {
-  const int c = threadIdx.x;
-  if (c >= 17) return;
-  float s = 0.f;
-  for (int k = 0; k < nb; k++) s += part[(size_t)k * 17 + c];
-  if (c < 16) gw[c] += s;
-  else gb[0] += s;
-}
 
 // --------------------------------------------------------- loss, optimiser
 // dout = scale * 2 (out - y); part[blk] = sum (out - y)^2 (FP64)
@@ -686,6 +726,19 @@ __global__ __launch_bounds__(256) void k_mse(const float *__restrict__ out, cons
     __syncthreads();
   }
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+}
+// *sum = the n (<= 1024) block partials of k_mse, in a fixed order
+__global__ __launch_bounds__(256) void k_mse_fold(const double *__restrict__ part, int n, double *__restrict__ sum) {
+  __shared__ double red[256];
+  double s = 0.0;
+  for (int k = threadIdx.x; k < n; k += 256) s += part[k];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *sum = red[0];
 }
 
 __global__ void k_adam(float *__restrict__ p, float *__restrict__ g, float *__restrict__ m, float *__restrict__ v,
@@ -808,27 +861,49 @@ void conv(const uint16_t *X, const uint16_t *W, const float *bias, uint16_t *Y, 
   HIPCHK(hipGetLastError());
 }
 
+// the partials of one backward pass: each layer's follow the last one's in
+// the buffer, all folded by one k_part_reduce
+struct Partials {
+  float *p;
+  size_t cap, used = 0;
+  RedJobs jobs{};
+  float *take(size_t n) {
+    if (used + n > cap) throw std::logic_error("gradient partials exceed their buffer");
+    float *r = p + used;
+    used += n;
+    return r;
+  }
+  void add(const float *part, float *g, int nparts, int cin, int cout, int taps) {
+    if (jobs.n == RED_JOBS) throw std::logic_error("too many gradient tensors");
+    jobs.j[jobs.n++] = RedJob{part, g, nparts, cin, cout, taps, jobs.blocks};
+    jobs.blocks += (cin * cout * taps + 63) / 64;
+  }
+  void fold(hipStream_t s) {
+    hipLaunchKernelGGL(k_part_reduce, dim3(jobs.blocks), dim3(256), 0, s, jobs);
+    HIPCHK(hipGetLastError());
+  }
+};
+
 template <int CIN, int COUT, int TAPS>
-void conv_dw(const uint16_t *X, const uint16_t *D, float *part, float *gw, int nx, int ny, int nz, hipStream_t s) {
+void conv_dw(const uint16_t *X, const uint16_t *D, Partials &P, float *gw, int nx, int ny, int nz, hipStream_t s) {
   const size_t N = (size_t)nx * ny * nz;
   const int ngroups = (int)((N + 255) / 256);
   const int nb = ngroups < 256 ? ngroups : 256;
+  float *part = P.take((size_t)TAPS * nb * 4 * CIN * COUT);
   hipLaunchKernelGGL((k_conv_dw<CIN, COUT, TAPS>), dim3(nb, TAPS), dim3(256), 0, s, X, D, part, nx, ny, nz);
   HIPCHK(hipGetLastError());
-  const int total = CIN * COUT * TAPS;
-  hipLaunchKernelGGL(k_dw_reduce, dim3((total + 255) / 256), dim3(256), 0, s, part, nb * 4, CIN, COUT, TAPS, gw);
-  HIPCHK(hipGetLastError());
+  P.add(part, gw, nb * 4, CIN, COUT, TAPS);
 }
 
 template <int C>
-void colsum(const uint16_t *D, size_t N, float *part, float *g, hipStream_t s) {
+void colsum(const uint16_t *D, size_t N, Partials &P, float *g, hipStream_t s) {
   constexpr int PER = 256 / C;
   size_t nb = (N + PER - 1) / PER;
   if (nb > 1024) nb = 1024;
+  float *part = P.take(nb * C);
   hipLaunchKernelGGL((k_colsum<C>), dim3((unsigned)nb), dim3(256), 0, s, D, N, part);
   HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_colsum_reduce, dim3(1), dim3(64), 0, s, part, (int)nb, C, g);
-  HIPCHK(hipGetLastError());
+  P.add(part, g, (int)nb, 1, C, 1);
 }
 
 void ew_launch_check() { HIPCHK(hipGetLastError()); }
@@ -921,8 +996,11 @@ void UNet::ensure(int nx, int ny, int nz, bool train) {
     A.g2a.alloc(N2 * 32); A.g2b.alloc(N2 * 32); A.g2c.alloc(N2 * 32);
     A.g3a.alloc(N3 * 64); A.g3b.alloc(N3 * 64);
     A.dout.alloc(N1);
-    // partials of the weight gradients: taps * 256 blocks * 4 waves * cin * cout
-    A.part.alloc((size_t)27 * 256 * 4 * 64 * 64);
+    // partials of every gradient tensor: at most 256 blocks of 4 waves per
+    // tap of the 3^3 weights and of the 1^3 ones, 1024 blocks per bias, 512
+    // of the head
+    A.part.alloc((size_t)27 * 1024 * (8 * 16 + 16 * 16 + 16 * 32 + 32 * 64 + 32 * 32 + 16 * 16) +
+                 (size_t)1024 * (64 * 32 + 32 * 16) + (size_t)1024 * (16 + 16 + 32 + 32 + 64 + 32 + 16 + 16) + 512 * 17);
   }
 }
 
@@ -978,13 +1056,16 @@ void UNet::backward(const uint16_t *X0, const float *dout, hipStream_t s) {
   const size_t N1 = (size_t)n1x * n1y * n1z, N2 = N1 / 8, N3 = N2 / 8;
   const uint16_t *W = Wp.p;
   const float *p = P.p;
-  float *g = G.p, *part = A.part.p;
+  float *g = G.p;
+  Partials part{A.part.p, A.part.n};
   // head
   {
     const unsigned nb = 512;
-    hipLaunchKernelGGL(k_head_bwd, dim3(nb), dim3(TPB), 0, s, A.a1.p, p + L[8].w, dout, A.g1a.p, N1, part);
-    hipLaunchKernelGGL(k_head_reduce, dim3(1), dim3(64), 0, s, part, (int)nb, g + L[8].w, g + L[8].b);
+    if (L[8].b != L[8].w + 16) throw std::logic_error("the head's bias follows its weights");
+    float *hp = part.take((size_t)nb * 17);
+    hipLaunchKernelGGL(k_head_bwd, dim3(nb), dim3(TPB), 0, s, A.a1.p, p + L[8].w, dout, A.g1a.p, N1, hp);
     ew_launch_check();
+    part.add(hp, g + L[8].w, (int)nb, 1, 17, 1);
   }
   // d1 (input t1, output a1; g1a = its masked output gradient)
   conv_dw<16, 16, 27>(A.t1.p, A.g1a.p, part, g + L[7].w, n1x, n1y, n1z, s);
@@ -1037,19 +1118,15 @@ void UNet::backward(const uint16_t *X0, const float *dout, hipStream_t s) {
   // e1 (no input gradient)
   conv_dw<8, 16, 27>(X0, A.g1a.p, part, g + L[0].w, n1x, n1y, n1z, s);
   colsum<16>(A.g1a.p, N1, part, g + L[0].b, s);
+  part.fold(s);
 }
 
-double UNet::loss_grad(const float *target, double scale, hipStream_t s) {
+void UNet::loss_grad(const float *target, double scale, double *sum, hipStream_t s) {
   const size_t N1 = (size_t)A.nx * A.ny * A.nz;
   const unsigned nb = 1024;
   hipLaunchKernelGGL(k_mse, dim3(nb), dim3(TPB), 0, s, A.out.p, target, N1, (float)scale, A.dout.p, A.red.p);
+  hipLaunchKernelGGL(k_mse_fold, dim3(1), dim3(256), 0, s, A.red.p, (int)nb, sum);
   HIPCHK(hipGetLastError());
-  std::vector<double> h(nb);
-  HIPCHK(hipMemcpyAsync(h.data(), A.red.p, sizeof(double) * nb, hipMemcpyDeviceToHost, s));
-  HIPCHK(hipStreamSynchronize(s));
-  double t = 0.0;
-  for (double x : h) t += x;
-  return t / (double)N1;
 }
 
 void UNet::adam(double lr, double b1, double b2, double eps, hipStream_t s) {
@@ -1290,19 +1367,29 @@ int phafd_unet_train(phafd_unet *u, int nsteps, int batch, int ntrain, double lr
     if (batch < 1 || ntrain < 1 || ntrain > n.ds_n) throw std::invalid_argument("bad batch or training range");
     n.ensure(n.ds_nx, n.ds_ny, n.ds_nz, true);
     const size_t N = (size_t)n.ds_nx * n.ds_ny * n.ds_nz;
+    // the samples' losses stay on the device until the last step: the host
+    // enqueues ahead instead of waiting for every sample
+    const size_t nl = (size_t)std::max(nsteps, 0) * batch;
+    n.losses.alloc(nl + 1);
     for (int k = 0; k < nsteps; k++) {
-      double lsum = 0.0;
       for (int b = 0; b < batch; b++) {
         const int idx = (int)(next_rand(n.rng) % (uint64_t)ntrain);
         const uint16_t *x = n.dsX.p + (size_t)idx * N * 8;
         n.forward(x, n.A.out.p, n.stream);
-        lsum += n.loss_grad(n.dsY.p + (size_t)idx * N, 1.0 / ((double)N * batch), n.stream);
+        n.loss_grad(n.dsY.p + (size_t)idx * N, 1.0 / ((double)N * batch), n.losses.p + (size_t)k * batch + b,
+                    n.stream);
         n.backward(x, n.A.dout.p, n.stream);
       }
       n.adam(lr, 0.9, 0.999, 1e-8, n.stream);
-      if (losses) losses[k] = lsum / batch;
     }
+    std::vector<double> h(nl);
+    if (nl) HIPCHK(hipMemcpyAsync(h.data(), n.losses.p, sizeof(double) * nl, hipMemcpyDeviceToHost, n.stream));
     HIPCHK(hipStreamSynchronize(n.stream));
+    for (int k = 0; losses && k < nsteps; k++) {
+      double t = 0.0;
+      for (int b = 0; b < batch; b++) t += h[(size_t)k * batch + b] / (double)N;
+      losses[k] = t / batch;
+    }
     return 0;
   });
 }
@@ -1314,11 +1401,15 @@ int phafd_unet_eval(phafd_unet *u, int i0, int count, double *losses) {
     if (i0 < 0 || count < 0 || i0 + count > n.ds_n) throw std::invalid_argument("sample range out of bounds");
     n.ensure(n.ds_nx, n.ds_ny, n.ds_nz, true);
     const size_t N = (size_t)n.ds_nx * n.ds_ny * n.ds_nz;
+    n.losses.alloc((size_t)count + 1);
     for (int k = 0; k < count; k++) {
       const uint16_t *x = n.dsX.p + (size_t)(i0 + k) * N * 8;
       n.forward(x, n.A.out.p, n.stream);
-      losses[k] = n.loss_grad(n.dsY.p + (size_t)(i0 + k) * N, 0.0, n.stream);
+      n.loss_grad(n.dsY.p + (size_t)(i0 + k) * N, 0.0, n.losses.p + k, n.stream);
     }
+    if (count) HIPCHK(hipMemcpyAsync(losses, n.losses.p, sizeof(double) * count, hipMemcpyDeviceToHost, n.stream));
+    HIPCHK(hipStreamSynchronize(n.stream));
+    for (int k = 0; k < count; k++) losses[k] /= (double)N;
     return 0;
   });
 }

@@ -56,6 +56,7 @@ struct UNet {
   DBuf<uint16_t> dsX;
   DBuf<float> dsY;
   int ds_n = 0, ds_nx = 0, ds_ny = 0, ds_nz = 0;
+  DBuf<double> losses;                   // one call's sums of squares, a sample each
   uint64_t rng = 0x9e3779b97f4a7c15ull;
   std::string err;
 
@@ -66,8 +67,8 @@ struct UNet {
   void forward(const uint16_t *X0, float *out, hipStream_t s);
   // gradients of sum_v dout[v] * out[v] added to G (after forward on the same input)
   void backward(const uint16_t *X0, const float *dout, hipStream_t s);
-  // mean square error of out against target, dout = its gradient times `scale`
-  double loss_grad(const float *target, double scale, hipStream_t s);
+  // *sum (device) = the sum of (out - target)^2, dout = its gradient times `scale`
+  void loss_grad(const float *target, double scale, double *sum, hipStream_t s);
   void adam(double lr, double b1, double b2, double eps, hipStream_t s);
 };
 

@@ -110,6 +110,29 @@ def test_parameter_gradients_match_torch_autograd():
     net.close()
 
 
+@pytest.mark.parametrize("shape", [(4, 32, 64), (12, 32, 64), (36, 64, 128)])
+def test_gradient_partials_of_every_count(shape):
+    """The fold of the gradients' partials where a layer has fewer than one
+    staged block of them (4 to 128), one and a part (384) and the most there
+    are (1024); the tolerance of the gradients above (bf16 gradients)."""
+    net = P.UNet(seed=3)
+    p = _random_params(net, 4)
+    net.set_params(p)
+    rng = np.random.default_rng(15)
+    x = rng.standard_normal((4,) + shape).astype(np.float32)
+    dout = (1.0 + 0.5 * rng.standard_normal(shape)).astype(np.float32)
+    net.forward(x)
+    net.backward(dout)
+    g = net.get_grads(zero=True)
+    tp = R.split_params(p, requires_grad=True)
+    (R.forward(tp, x) * torch.as_tensor(dout)).sum().backward()
+    gr = R.flat_grads(tp)
+    for name, ws, bs in _layer_slices():
+        assert rel_l2(g[ws], gr[ws]) < 3e-2, f"{name} weight grad"
+        assert rel_l2(g[bs], gr[bs]) < 3e-2, f"{name} bias grad"
+    net.close()
+
+
 def test_gradients_against_finite_differences():
     net = P.UNet(seed=3)
     p = _random_params(net, 7)
