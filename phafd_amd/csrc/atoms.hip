@@ -618,28 +618,6 @@ struct MuAcc<float> {
   }
   __device__ __forceinline__ float get() const { return m; }
 };
-// running force of one atom: FP64 subtracts each term from F in order; FP32
-// sums the terms with Kahan compensation and subtracts the sum once
-template <class R>
-struct ForceAcc {
-  double4 F;
-  __device__ __forceinline__ void sub(double fx, double fy, double fz) { F.x -= fx; F.y -= fy; F.z -= fz; }
-  __device__ __forceinline__ double4 get() const { return F; }
-};
-template <>
-struct ForceAcc<float> {
-  double4 F;
-  Kahan kx, ky, kz;
-  __device__ __forceinline__ void sub(float fx, float fy, float fz) { kx.add(fx); ky.add(fy); kz.add(fz); }
-  __device__ __forceinline__ double4 get() const {
-    double4 r = F;
-    r.x -= (double)kx.s;
-    r.y -= (double)ky.s;
-    r.z -= (double)kz.s;
-    return r;
-  }
-};
-
 // the kernel value e of one in-cut pair (rsq already divided by cutsq): the
 // expressions of the reference's loops; FP32 form: rsq in FP64 from the FP64
 // positions, e in FP32
@@ -694,6 +672,32 @@ __global__ void k_ga_am_walk(int ng, GridView gv, const double4 *__restrict__ gx
       }
     }
     if (!off) cnt[q] = n;
+  }
+}
+// The order the force walk takes the atoms in: tiles of GA_TILE^3 bins, z
+// major, the bins' own order within a tile.  Bin order runs through whole
+// planes of bins, so by the time the walk returns to a point's neighbourhood
+// one plane later its field lines and its half-written lines of mu terms have
+// left the 4 MB L2; a tile's stay.  row = one x run of GA_TILE bins of one
+// tile; FILL: its atoms go to perm[off[row]...), else their number to cnt[row].
+constexpr int GA_TILE = 8;
+template <bool FILL>
+__global__ __launch_bounds__(256) void k_ga_tile_rows(int nrow, int ntx, int nty, BinGeom bg,
+                                                      const int *__restrict__ binstart, int *__restrict__ cnt,
+                                                      const int *__restrict__ off, int *__restrict__ perm) {
+  GRID_STRIDE(r, nrow) {
+    const int ry = (int)r % GA_TILE, rz = (int)r / GA_TILE % GA_TILE, t = (int)r / (GA_TILE * GA_TILE);
+    const int tx = t % ntx, ty = t / ntx % nty, tz = t / ntx / nty;
+    const int y = ty * GA_TILE + ry, z = tz * GA_TILE + rz;
+    int b = 0, e = 0;
+    if (y < bg.mbiny && z < bg.mbinz) {
+      const int row = (z * bg.mbiny + y) * bg.mbinx, x1 = (tx + 1) * GA_TILE;
+      b = binstart[row + tx * GA_TILE];
+      e = binstart[row + (x1 < bg.mbinx ? x1 : bg.mbinx)];
+    }
+    if (!FILL) cnt[r] = e - b;
+    else
+      for (int q = b, w = off[r]; q < e; q++, w++) perm[w] = q;
   }
 }
 // per pair: its rank among its point's pairs (arbitrary), and the point count
@@ -781,109 +785,146 @@ __global__ __launch_bounds__(256) void k_ga_pm_sort(size_t N, const int *__restr
   }
 }
 
-// The step's grid-atom pass, atom side: one thread per atom (bin order q)
-// walks its build pairs in ascending grid index, keeps those in the pair
-// cut now (the reference's test), and subtracts their force terms in that
-// order.  The mu term of each pair it keeps goes to its grid point's slot,
-// mterm[ps[entry].y] (NaN for a pair out of the cut).  Entries are taken
-// GA_B at a time: the tests and field loads first, then the terms in
-// order, so that up to GA_B pairs' loads are in flight.  Grid sides are
+// The step's grid-atom pass, atom side: G lanes per atom (bin order q) take
+// its build pairs G at a time in ascending grid index, keep those in the pair
+// cut now (the reference's test) and form their terms; the mu term of each
+// kept pair goes to its grid point's slot, mterm[ps[entry].y] (NaN for a pair
+// out of the cut).  The force terms go through LDS to three of the G lanes,
+// one per component, which subtract them in ascending grid index: the sums
+// are those of a plain loop over the pairs, bit for bit.  Grid sides are
 // powers of two (lx = log2 nx, lxy = log2 (nx ny)).
-constexpr int GA_B = 8;
-// the force walk of gathered atom number q of the bin-sorted order (ZI: gF
-// starts from zero instead of its stored value, and atoms without pairs
-// get zero written -- the fill and the walk in one)
-template <class R, bool ZI>
-__device__ __forceinline__ void ga_force_atom(size_t q, const GridViewT<R> &gv, const GAParams &ga,
+// With a thread per atom every load touched 64 atoms' unrelated lines and the
+// walk was bound by L1 and L2 traffic (a line per 8-byte value); G lanes of
+// one atom share the lines of its x runs.  Thread per atom -> now, us a
+// launch: 161 -> 109 (256^3 FP64, 500k beads, 8 pairs per atom), 6894 -> 2544
+// (512^3 FP32, 2M beads, 87 pairs per atom), 287 -> 104 (512 x 128 x 32 FP64,
+// 63k beads, 87).  What bounds the wide case now: about half the cycles issue
+// arithmetic, and the mu terms' scattered 4-byte stores leave L2 as 45M
+// 64-byte writes, four times the terms' bytes.
+template <class R> struct GAShared { R t[3][66]; };   // one wave's terms, a row per component
+// One component of one atom's force.  FP64 subtracts each term in order (a
+// pair out of the cut leaves a zero: the same sum).  FP32 sums the terms with
+// Kahan compensation and subtracts the sum once; there a zero term would move
+// the compensation, so the kept terms stand packed at the front instead.
+template <class R>
+struct ForceSum {
+  static constexpr bool PACKED = false;
+  double F;
+  __device__ __forceinline__ void sub(double v) { F -= v; }
+  __device__ __forceinline__ double get() const { return F; }
+};
+template <>
+struct ForceSum<float> {
+  static constexpr bool PACKED = true;
+  double F;
+  Kahan k;
+  __device__ __forceinline__ void sub(float v) { k.add(v); }
+  __device__ __forceinline__ double get() const { return F - (double)k.s; }
+};
+// the force of gathered atom number q of the bin-sorted order (ZI: gF starts
+// from zero instead of its stored value -- the fill and the walk in one).
+// Every lane of the wave calls it; lanes without an atom pass on = false.
+template <class R, bool ZI, int G>
+__device__ __forceinline__ void ga_force_atom(size_t q, bool on, const GridViewT<R> &gv, const GAParams &ga,
                                               const double4 *__restrict__ gx, const int *__restrict__ order,
                                               const int *__restrict__ aoff, const int2 *__restrict__ ps,
-                                              R *__restrict__ mterm, double4 *__restrict__ gF, double &esum,
-                                              bool want_energy, int lx, int lxy) {
+                                              R *__restrict__ mterm, double4 *__restrict__ gF, GAShared<R> &sh,
+                                              double &esum, bool want_energy, int lx, int lxy) {
   const int mx = gv.nx - 1, my = gv.ny - 1;
-  const int s = aoff[q], e = aoff[q + 1];
-  const int a = order[q];
-  if (s == e) {
-    if (ZI) gF[a] = make_double4(0.0, 0.0, 0.0, 0.0);
-    return;
+  const int lane = threadIdx.x & 63, sub = lane & (G - 1), first = lane & ~(G - 1);
+  int c = 0, e = 0, a = 0;
+  if (on) {
+    c = aoff[q] + sub;
+    e = aoff[q + 1];
+    a = order[q];
   }
-  const double4 x = gx[a];
-  const double4 F0 = ZI ? make_double4(0.0, 0.0, 0.0, 0.0) : gF[a];
+  int2 nx = c < e ? ps[c] : make_int2(0, 0);
+  double4 x = make_double4(0.0, 0.0, 0.0, 0.0);
+  if (on) x = gx[a];
   const int t = (int)x.w;
   const double cs = ga.cutsq[t];
   const R phit = (R)ga.phit[t];
-  ForceAcc<R> acc;
-  acc.F = F0;
-  bool any = false;
-  // the pair entries of the next batch load while this batch's grid
-  // values load and its terms are formed
-  int2 nx[GA_B];
-#pragma unroll
-  for (int u = 0; u < GA_B; u++) nx[u] = s + u < e ? ps[s + u] : make_int2(0, 0);
-  for (int c0 = s; c0 < e; c0 += GA_B) {
-    int pp[GA_B], so[GA_B];
-#pragma unroll
-    for (int u = 0; u < GA_B; u++) {
-      pp[u] = nx[u].x;
-      so[u] = nx[u].y;
-    }
-#pragma unroll
-    for (int u = 0; u < GA_B; u++) nx[u] = c0 + GA_B + u < e ? ps[c0 + GA_B + u] : make_int2(0, 0);
-    bool in[GA_B];
-    double rs[GA_B];
-    R ph[GA_B], fx[GA_B], fy[GA_B], fz[GA_B];
-#pragma unroll
-    for (int u = 0; u < GA_B; u++) {
-      const int p = pp[u];
-      const int k = p & mx, j = (p >> lx) & my, i = p >> lxy;
-      const double delz = (i * gv.dz + gv.lo[2]) - x.z;
-      const double dely = (j * gv.dy + gv.lo[1]) - x.y;
-      const double delx = (k * gv.dx + gv.lo[0]) - x.x;
-      const double rsq = delx * delx + dely * dely + delz * delz;
-      in[u] = c0 + u < e && ga_in(ga, rsq, cs);   // NaN positions: false
-      rs[u] = rsq;
-      ph[u] = fx[u] = fy[u] = fz[u] = R(0);
-      if (in[u]) {
-        ph[u] = gv.phi[p];
-        fx[u] = gv.gx[p];
-        fy[u] = gv.gy[p];
-        fz[u] = gv.gz[p];
-      } else if (c0 + u < e) {
-        mterm[so[u]] = __builtin_nan("");
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < GA_B; u++) {
-      if (!in[u]) continue;
-      R expfac = ga_expfac<R>(ga, rs[u] / cs, t);
+  double *Fa = reinterpret_cast<double *>(gF + a);
+  ForceSum<R> acc;
+  acc.F = 0.0;
+  if (!ZI && on && sub < 3) acc.F = Fa[sub];
+  while (__any(c < e)) {
+    const bool act = c < e;
+    const int p = nx.x, so = nx.y;
+    c += G;
+    nx = c < e ? ps[c] : make_int2(0, 0);   // the next pairs load while these terms are formed
+    const int k = p & mx, j = (p >> lx) & my, i = p >> lxy;
+    const double delz = (i * gv.dz + gv.lo[2]) - x.z;
+    const double dely = (j * gv.dy + gv.lo[1]) - x.y;
+    const double delx = (k * gv.dx + gv.lo[0]) - x.x;
+    const double rsq = delx * delx + dely * dely + delz * delz;
+    const bool in = act && ga_in(ga, rsq, cs);   // NaN positions: false
+    R tx = R(0), ty = R(0), tz = R(0);
+    if (in) {
+      const R ph = gv.phi[p], fx = gv.gx[p], fy = gv.gy[p], fz = gv.gz[p];
+      R expfac = ga_expfac<R>(ga, rsq / cs, t);
       if (ga.style == GA_LJISH_LINEAR) {
         // PairGridAtomLJishLinear::compute (src/pair_gridatom_lj_ish_linear.cpp:
         // 93-160): e = -1 * bump * eps, mu += e, force weight e dv, no energy
         expfac = -expfac;
-        mterm[so[u]] = expfac;
+        mterm[so] = expfac;
         expfac *= (R)gv.dv;
       } else {
-        const R delphi = (ph[u] - phit);
-        mterm[so[u]] = 2 * delphi * expfac;
+        const R delphi = (ph - phit);
+        mterm[so] = 2 * delphi * expfac;
         if (want_energy) esum += (double)delphi * (double)delphi * (double)expfac * gv.dv;
         expfac *= 2 * delphi * (R)gv.dv;
       }
-      acc.sub(fx[u] * expfac, fy[u] * expfac, fz[u] * expfac);
-      any = true;
+      tx = fx * expfac;
+      ty = fy * expfac;
+      tz = fz * expfac;
+    } else if (act) {
+      mterm[so] = __builtin_nan("");
     }
+    int slot = lane, n = G;
+    if constexpr (ForceSum<R>::PACKED) {
+      const unsigned long long kept = __ballot(in) & ((unsigned long long)((1u << G) - 1) << first);
+      slot = first + __builtin_amdgcn_mbcnt_hi((unsigned)(kept >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)kept, 0u));
+      n = __popcll(kept);
+    }
+    if (in || !ForceSum<R>::PACKED) {
+      sh.t[0][slot] = tx;
+      sh.t[1][slot] = ty;
+      sh.t[2][slot] = tz;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (sub < 3) {
+#pragma unroll
+      for (int h = 0; h < G; h += 8) {   // eight terms' reads in flight
+        R v[8];
+#pragma unroll
+        for (int u = 0; u < 8 && h + u < G; u++) v[u] = sh.t[sub][first + h + u];
+#pragma unroll
+        for (int u = 0; u < 8 && h + u < G; u++)
+          if (!ForceSum<R>::PACKED || h + u < n) acc.sub(v[u]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
-  if (any || ZI) gF[a] = acc.get();
+  if (on && sub < 3) Fa[sub] = acc.get();
+  if (ZI && on && sub == 3) Fa[3] = 0.0;
 }
 
-template <class R>
+template <class R, int G>
 __global__ __launch_bounds__(256) void k_ga_force(int ng, GridViewT<R> gv, GAParams ga,
                                                   const double4 *__restrict__ gx, const int *__restrict__ order,
-                                                  const int *__restrict__ aoff, const int2 *__restrict__ ps,
-                                                  R *__restrict__ mterm,
+                                                  const int *__restrict__ perm, const int *__restrict__ aoff,
+                                                  const int2 *__restrict__ ps, R *__restrict__ mterm,
                                                   double4 *__restrict__ gF, double *energy, int lx, int lxy) {
+  __shared__ GAShared<R> sh[4];
   double esum = 0.0;
-  const size_t bl = xcd_block(blockIdx.x, gridDim.x);
-  for (size_t q = bl * blockDim.x + threadIdx.x; q < (size_t)ng; q += (size_t)gridDim.x * blockDim.x)
-    ga_force_atom<R, false>(q, gv, ga, gx, order, aoff, ps, mterm, gF, esum, energy != nullptr, lx, lxy);
+  const size_t i = (size_t)xcd_block(blockIdx.x, gridDim.x) * (256 / G) + threadIdx.x / G;
+  const bool on = i < (size_t)ng;
+  const size_t q = perm && on ? (size_t)perm[i] : i;
+  ga_force_atom<R, false, G>(q, on, gv, ga, gx, order, aoff, ps, mterm, gF, sh[threadIdx.x / 64], esum,
+                             energy != nullptr, lx, lxy);
   if (energy && esum != 0.0) atomicAdd(energy, esum);
 }
 
@@ -898,19 +939,23 @@ __device__ __forceinline__ int member_of(const int *__restrict__ boff, int nm, i
   return lo;
 }
 
-// every member's force walk in one launch: item = a block of 256 gathered
-// atoms of one member, items taken round-robin by a grid of at most a few
-// blocks per CU (gF written from zero: the fill folded in)
+// every member's force walk in one launch: item = as many gathered atoms of
+// one member as the block has threads, G lanes each, items taken round-robin
+// by a grid of at most a few blocks per CU (gF written from zero: the fill
+// folded in)
+template <int G>
 __global__ __launch_bounds__(256) void k_ga_force_multi(const GAMemberDev *__restrict__ d,
                                                         const int *__restrict__ boff, int nm, int lx, int lxy) {
+  __shared__ GAShared<double> sh[4];
   const int nitems = boff[nm];
   for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
     const int m = member_of(boff, nm, item);
     const GAMemberDev &g = d[m];
-    const size_t q = (size_t)(item - boff[m]) * blockDim.x + threadIdx.x;
+    const size_t q0 = (size_t)(item - boff[m]) * blockDim.x + threadIdx.x / G;
     double esum = 0.0;
-    if (q < (size_t)g.ng)
-      ga_force_atom<double, true>(q, g.gv, g.ga, g.gx, g.order, g.aoff, g.ps, g.mterm, g.gF, esum, false, lx, lxy);
+    for (unsigned r = 0; r < blockDim.x; r += blockDim.x / G)
+      ga_force_atom<double, true, G>(q0 + r, q0 + r < (size_t)g.ng, g.gv, g.ga, g.gx, g.order, g.aoff, g.ps, g.mterm,
+                                     g.gF, sh[threadIdx.x / 64], esum, false, lx, lxy);
   }
 }
 
@@ -1851,6 +1896,21 @@ void launch_ga_am_walk(int ng, const GridView &gv, const double4 *gxb, const int
   hipLaunchKernelGGL(k_ga_am_walk, dim3(nblk(ng)), dim3(TPB), 0, s, ng, gv, gxb, order, reachsq, cnt, off, ps, amq);
   HIPCHK(hipGetLastError());
 }
+int64_t ga_tile_rows(const BinGeom &bg) {
+  auto nt = [](int m) { return ((int64_t)m + GA_TILE - 1) / GA_TILE; };
+  return nt(bg.mbinx) * nt(bg.mbiny) * nt(bg.mbinz) * GA_TILE * GA_TILE;
+}
+void launch_ga_tile_rows(bool fill, const BinGeom &bg, const int *binstart, int *cnt, const int *off, int *perm,
+                         hipStream_t s) {
+  const int nrow = (int)ga_tile_rows(bg), ntx = (bg.mbinx + GA_TILE - 1) / GA_TILE, nty = (bg.mbiny + GA_TILE - 1) / GA_TILE;
+  if (fill)
+    hipLaunchKernelGGL(k_ga_tile_rows<true>, dim3(nblk(nrow)), dim3(TPB), 0, s, nrow, ntx, nty, bg, binstart, cnt, off,
+                       perm);
+  else
+    hipLaunchKernelGGL(k_ga_tile_rows<false>, dim3(nblk(nrow)), dim3(TPB), 0, s, nrow, ntx, nty, bg, binstart, cnt,
+                       off, perm);
+  HIPCHK(hipGetLastError());
+}
 void launch_ga_pm_count(int nent, const int2 *ps, int *pcnt, int *rank, hipStream_t s) {
   if (nent <= 0) return;
   hipLaunchKernelGGL(k_ga_pm_count, dim3(nblk(nent)), dim3(TPB), 0, s, nent, ps, pcnt, rank);
@@ -1872,13 +1932,25 @@ static int ilog2(int v) {
   if ((1 << l) != v) throw std::invalid_argument("grid sides must be powers of two");
   return l;
 }
+// Lanes per atom of the force walk and the order of its atoms.  16 lanes cover
+// a wide coupling's x runs (5 points at reach 2.75) with fewer cache lines per
+// load, 8 leave fewer lanes idle on a narrow one's few pairs.  Measured, us a
+// launch (8 lanes / 16 lanes / 16 lanes by tiles): 87 pairs per atom, 512^3
+// FP32, 2M beads 3820 / 3067 / 2544 and 512 x 128 x 32 FP64 151 / 131 / 104;
+// 8 pairs per atom, 256^3 FP64, 500k beads 109 / 136 / 139 (8 lanes by tiles:
+// 108, not worth the order's build).  48 pairs per atom (reach 2.25, 128^3):
+// 16 lanes 4% less per step.  24 pairs, three rounds of 8 lanes, is between.
+bool ga_wide(int64_t ng, int64_t nent) { return nent >= 24 * ng; }
 #define PHAFD_GA_DEF(RT)                                                                                        \
-  void launch_ga_force(int ng, const GridViewT<RT> &gv, const GAParams &ga, const double4 *gx, const int *order, \
-                       const int *aoff, const int2 *ps, RT *mterm, double4 *gF, double *energy, hipStream_t s) { \
+  void launch_ga_force(int ng, int64_t nent, const GridViewT<RT> &gv, const GAParams &ga, const double4 *gx,   \
+                       const int *order, const int *perm, const int *aoff, const int2 *ps, RT *mterm, double4 *gF, \
+                       double *energy, hipStream_t s) {                                                       \
     if (ng <= 0) return;                                                                                      \
     const int lx = ilog2(gv.nx), lxy = lx + ilog2(gv.ny);                                                     \
-    hipLaunchKernelGGL(k_ga_force<RT>, dim3(nblk(ng)), dim3(TPB), 0, s, ng, gv, ga, gx, order, aoff, ps,      \
-                       mterm, gF, energy, lx, lxy);                                                           \
+    const int G = ga_wide(ng, nent) ? 16 : 8;                                                                 \
+    const auto k = G == 16 ? k_ga_force<RT, 16> : k_ga_force<RT, 8>;                                          \
+    hipLaunchKernelGGL(k, dim3((unsigned)(((size_t)ng * G + 255) / 256)), dim3(256), 0, s, ng, gv, ga, gx,    \
+                       order, perm, aoff, ps, mterm, gF, energy, lx, lxy);                                    \
     HIPCHK(hipGetLastError());                                                                                \
   }                                                                                                           \
   void launch_ga_list_mu(size_t N, RT *mu, const int *poff, const RT *mterm, bool first, hipStream_t s) {     \
@@ -1961,13 +2033,13 @@ void check_shape(const MultiShape &sh) {
   if ((sh.threads != 64 && sh.threads != 128 && sh.threads != 256) || sh.cap < 1)
     throw std::invalid_argument("batched pair phase: items of 64, 128 or 256 atoms, a positive grid cap");
 }
-void launch_ga_force_multi(int nm, const GAMemberDev *d, const int *boff, int nitems, int nx, int ny,
+void launch_ga_force_multi(int nm, const GAMemberDev *d, const int *boff, int nitems, bool wide, int nx, int ny,
                            const MultiShape &sh, hipStream_t s) {
   if (nm <= 0 || nitems <= 0) return;
   check_shape(sh);
   const int lx = ilog2(nx), lxy = lx + ilog2(ny);
-  hipLaunchKernelGGL(k_ga_force_multi, dim3(multi_grid(nitems, sh.cap)), dim3(sh.threads), 0, s, d, boff, nm, lx,
-                     lxy);
+  hipLaunchKernelGGL(wide ? k_ga_force_multi<16> : k_ga_force_multi<8>, dim3(multi_grid(nitems, sh.cap)),
+                     dim3(sh.threads), 0, s, d, boff, nm, lx, lxy);
   HIPCHK(hipGetLastError());
 }
 void launch_ga_list_mu_multi(int nm, size_t N, const GAMemberDev *d, hipStream_t s) {

@@ -119,19 +119,27 @@ void launch_ga_density(int ng, const GridView &gv, const GAParams &ga, const dou
 // scan; key, ent scratch): ps[entry].y = its slot in the point's segment.
 void launch_ga_am_walk(int ng, const GridView &gv, const double4 *gxb, const int *order, double reachsq, int *cnt,
                        const int *off, int2 *ps, int *amq, hipStream_t s);
+// a wide coupling: many pairs per gathered atom (the force walk's shape)
+bool ga_wide(int64_t ng, int64_t nent);
+// the atoms (bin order positions q) tile by tile, a wide walk's order:
+// rows of a build, their counts (fill = false) and contents
+int64_t ga_tile_rows(const BinGeom &bg);
+void launch_ga_tile_rows(bool fill, const BinGeom &bg, const int *binstart, int *cnt, const int *off, int *perm,
+                         hipStream_t s);
 void launch_ga_pm_count(int nent, const int2 *ps, int *pcnt, int *rank, hipStream_t s);
 void launch_ga_pm_place(int nent, int2 *ps, const int *rank, const int *amq, const int *poff, int *key, int *ent,
                         size_t N, hipStream_t s);
 // One grid-atom pair style (PairGridAtomGaussian / LJish / LJish/linear
-// compute) over the pairs of the last build.  launch_ga_force: gF(a) -= the
+// compute) over the nent pairs of the last build.  launch_ga_force: gF(a) -= the
 // atom's terms in ascending grid index (FP32 form: Kahan-summed FP32 terms
 // subtracted once); mterm[ps[entry].y] = the pair's mu term, NaN out of the
 // cut; energy (may be null) += the coupling energy.
 // launch_ga_list_mu: mu(g) (first: from zero, else added to) += the terms
 // of its segment in order (ascending q, the reference's order).
 #define PHAFD_GA_DECL(RT)                                                                                       \
-  void launch_ga_force(int ng, const GridViewT<RT> &gv, const GAParams &ga, const double4 *gx, const int *order, \
-                       const int *aoff, const int2 *ps, RT *mterm, double4 *gF, double *energy, hipStream_t s);  \
+  void launch_ga_force(int ng, int64_t nent, const GridViewT<RT> &gv, const GAParams &ga, const double4 *gx,     \
+                       const int *order, const int *perm, const int *aoff, const int2 *ps, RT *mterm,           \
+                       double4 *gF, double *energy, hipStream_t s);                                             \
   void launch_ga_list_mu(size_t N, RT *mu, const int *poff, const RT *mterm, bool first, hipStream_t s);
 PHAFD_GA_DECL(double)
 PHAFD_GA_DECL(float)
@@ -201,7 +209,7 @@ struct MultiShape {
   int threads = 256, cap = 2048;
 };
 // gF of every gathered atom written (from zero: the fill folded in)
-void launch_ga_force_multi(int nm, const GAMemberDev *d, const int *boff, int nitems, int nx, int ny,
+void launch_ga_force_multi(int nm, const GAMemberDev *d, const int *boff, int nitems, bool wide, int nx, int ny,
                            const MultiShape &sh, hipStream_t s);
 void launch_ga_list_mu_multi(int nm, size_t N, const GAMemberDev *d, hipStream_t s);
 void launch_lj_multi(int nm, const LJMemberDev *d, const int *boff, int nitems, const MultiShape &sh,

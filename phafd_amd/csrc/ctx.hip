@@ -179,6 +179,8 @@ struct phafd_hip_ctx {
   // the reference's list order, ascending q (ga_poff; ga_ps.y: the
   // atom-major entry's slot); ga_mterm: each slot's mu term of the current
   // pass (NaN out of the cut)
+  DBuf<int> ga_tcnt, ga_toff, ga_perm;   // wide couplings: the atoms in tile order
+  bool ga_tiled = false;
   DBuf<int> ga_acnt, ga_aoff, ga_amq, ga_rank, ga_pcnt, ga_poff, ga_key, ga_ent;
   DBuf<int2> ga_ps;
   DBuf<double> ga_mterm;
@@ -708,6 +710,16 @@ void build_ga_pairs(phafd_hip_ctx *c) {
   const int nent = read_int(c, c->ga_aoff.p + ng);
   if (nent < 0) throw std::runtime_error("grid-atom pairs of a build exceed 2^31");
   c->ga_nent = nent;
+  const int64_t nrow = ga_tile_rows(c->bg);
+  c->ga_tiled = ga_wide(ng, nent) && nrow < INT32_MAX;
+  if (c->ga_tiled) {   // the force walk takes the atoms tile by tile
+    c->ga_tcnt.alloc((size_t)nrow + 1);
+    c->ga_toff.alloc((size_t)nrow + 2);
+    c->ga_perm.alloc((size_t)ng + 1);
+    launch_ga_tile_rows(false, c->bg, c->binstart.p, c->ga_tcnt.p, nullptr, nullptr, c->stream);
+    scan_exclusive_i32(c->ga_tcnt.p, c->ga_toff.p, (size_t)nrow, c->stream);
+    launch_ga_tile_rows(true, c->bg, c->binstart.p, nullptr, c->ga_toff.p, c->ga_perm.p, c->stream);
+  }
   c->ga_ps.alloc((size_t)nent + 1);
   c->ga_amq.alloc((size_t)nent + 1);
   launch_ga_am_walk(ng, gv, c->gx_build.p, c->binatoms.p, reach * reach, nullptr, c->ga_aoff.p, c->ga_ps.p,
@@ -951,8 +963,8 @@ void grid_atom_pass(phafd_hip_ctx *c, PairDef &p, double *energy, bool first) {
   // algorithmic bytes: phi and its gradient read once (4 fields), each
   // gathered atom's position read and force written
   probe_begin(K_GA_FORCE, c->stream);
-  launch_ga_force(c->ngathered, gvr, ga, c->gx.p, c->binatoms.p, c->ga_aoff.p, c->ga_ps.p, mt.p, c->gF.p, energy,
-                  c->stream);
+  launch_ga_force(c->ngathered, c->ga_nent, gvr, ga, c->gx.p, c->binatoms.p, c->ga_tiled ? c->ga_perm.p : nullptr,
+                  c->ga_aoff.p, c->ga_ps.p, mt.p, c->gF.p, energy, c->stream);
   probe_end(K_GA_FORCE, c->stream, 4.0 * sizeof(R) * c->N + 64.0 * c->ngathered);
   probe_begin(K_GA_DEPOSIT, c->stream);
   if (!(c->eager_gridlist && c->grid_built)) {
@@ -3158,9 +3170,12 @@ void batch_pair_fused(phafd_hip_batch *b, bool with_chains) {
   const int *di = (const int *)(d + P.off_int);
   const int *dboff_ga = di, *dboff_fold = di + stride, *dcoff = dboff_fold + (size_t)stride * (P.nlev + 1);
   double ng_all = 0;
+  int64_t nent_all = 0;
   for (auto &g : ga) ng_all += g.ng;
+  for (auto &m : b->members) nent_all += m->ga_nent;
   probe_begin(K_GA_FORCE, b->stream);
-  launch_ga_force_multi(nm, dga, dboff_ga, P.items_ga, c0->nx, c0->ny, b->shape, b->stream);
+  launch_ga_force_multi(nm, dga, dboff_ga, P.items_ga, ga_wide((int64_t)ng_all, nent_all), c0->nx, c0->ny,
+                        b->shape, b->stream);
   probe_end(K_GA_FORCE, b->stream, 4.0 * sizeof(double) * b->N * nm + 64.0 * ng_all);
   launch_ga_list_mu_multi(nm, b->N, dga, b->stream);
   if (P.lj) launch_lj_multi(nm, dlj, dboff_ga, P.items_ga, b->shape, b->stream);
