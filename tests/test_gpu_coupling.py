@@ -20,7 +20,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("nchains,nbeads", [(1, 1), (1, 7), (9, 15)])
 def test_force_walk_shapes(style, width, nchains, nbeads):
     w = workload(n=32, nchains=nchains, nbeads=nbeads, ljish=style, nucwidth=width, gauss_cut=3.0, zghost=1,
-                 seed=31, types=2, chain=nbeads > 1)
+                 seed=31, types=2 if nbeads > 1 else 1, chain=nbeads > 1)
     g, o = make_gpu(w), make_oracle(w)
     e = make_gpu(w)
     e.set_option(P.OPT_EAGER_GRIDLIST, 1)
