@@ -234,6 +234,7 @@ struct phafd_hip_ctx {
   DBuf<int> sg_img;
   DumpJob dump[2];   // [0] grid, [1] atoms: the two kinds write concurrently
   DBuf<double4> cp_keep;   // owned forces kept across a compute pair
+  DBuf<double> conv;       // stage of a host array converted on the device
 
   double dx() const { return period[0] / nx; }   // src/grid.cpp:187-201
   double dy() const { return period[1] / ny; }
@@ -1499,16 +1500,31 @@ R *field_ptr(phafd_hip_ctx *c, int which) {
   throw std::invalid_argument("unknown field");
 }
 
-// the host side always holds FP64; the FP32 form rounds on the way in
+// The host side always holds FP64.  The FP32 form converts on the device, a
+// chunk at a time through a bounded stage (64 MB).  Converting on the host was
+// one core's loop behind a copy into a zeroed vector: reading phi, positions
+// and forces took 21 ms longer at 256^3 / 500k beads, 175 ms at 512^3 / 2M.
+constexpr size_t CONV_CHUNK = (size_t)8 << 20;   // values
+__global__ void k_widen_field(size_t n, const float *__restrict__ a, double *__restrict__ b) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    b[i] = (double)a[i];
+}
+__global__ void k_narrow_field(size_t n, const double *__restrict__ a, float *__restrict__ b) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    b[i] = (float)a[i];
+}
 void field_in(phafd_hip_ctx *c, int which, const double *h) {
   if (!c->fp32) {
     HIPCHK(hipMemcpyAsync(field_ptr<double>(c, which), h, sizeof(double) * c->N, hipMemcpyHostToDevice, c->stream));
   } else {
-    std::vector<float> t(c->N);
-    for (size_t i = 0; i < c->N; i++) t[i] = (float)h[i];
-    HIPCHK(hipMemcpyAsync(field_ptr<float>(c, which), t.data(), sizeof(float) * c->N, hipMemcpyHostToDevice,
-                          c->stream));
-    sync(c);
+    c->conv.alloc(std::min(c->N, CONV_CHUNK));
+    for (size_t o = 0; o < c->N; o += CONV_CHUNK) {
+      const size_t n = std::min(CONV_CHUNK, c->N - o);
+      HIPCHK(hipMemcpyAsync(c->conv.p, h + o, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+      hipLaunchKernelGGL(k_narrow_field, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, c->stream, n, c->conv.p,
+                         field_ptr<float>(c, which) + o);
+      HIPCHK(hipGetLastError());
+    }
   }
   sync(c);
 }
@@ -1517,11 +1533,15 @@ void field_out(phafd_hip_ctx *c, int which, double *h) {
     HIPCHK(hipMemcpyAsync(h, field_ptr<double>(c, which), sizeof(double) * c->N, hipMemcpyDeviceToHost, c->stream));
     sync(c);
   } else {
-    std::vector<float> t(c->N);
-    HIPCHK(hipMemcpyAsync(t.data(), field_ptr<float>(c, which), sizeof(float) * c->N, hipMemcpyDeviceToHost,
-                          c->stream));
+    c->conv.alloc(std::min(c->N, CONV_CHUNK));
+    for (size_t o = 0; o < c->N; o += CONV_CHUNK) {
+      const size_t n = std::min(CONV_CHUNK, c->N - o);
+      hipLaunchKernelGGL(k_widen_field, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, c->stream, n,
+                         field_ptr<float>(c, which) + o, c->conv.p);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipMemcpyAsync(h + o, c->conv.p, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
+    }
     sync(c);
-    for (size_t i = 0; i < c->N; i++) h[i] = t[i];
   }
 }
 
@@ -1530,12 +1550,22 @@ std::vector<double4> to_d4(const double *xyz, int n) {
   for (int i = 0; i < n; i++) v[i] = make_double4(xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], 0.0);
   return v;
 }
-void from_d4(const std::vector<double4> &v, double *xyz) {
-  for (size_t i = 0; i < v.size(); i++) {
-    xyz[3 * i] = v[i].x;
-    xyz[3 * i + 1] = v[i].y;
-    xyz[3 * i + 2] = v[i].z;
+// n device vectors to the host as n rows of three, packed on the device: the
+// fourth component stays there and the host loops over nothing
+__global__ void k_pack3(size_t n, const double4 *__restrict__ a, double *__restrict__ b) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < 3 * n; i += (size_t)gridDim.x * blockDim.x)
+    b[i] = reinterpret_cast<const double *>(a)[i / 3 * 4 + i % 3];
+}
+void download3(phafd_hip_ctx *c, const double4 *d, size_t n, double *xyz) {
+  const size_t most = CONV_CHUNK / 3;
+  c->conv.alloc(3 * std::min(n, most));
+  for (size_t o = 0; o < n; o += most) {
+    const size_t m = std::min(most, n - o);
+    hipLaunchKernelGGL(k_pack3, dim3((unsigned)((3 * m + 255) / 256)), dim3(256), 0, c->stream, m, d + o, c->conv.p);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(xyz + 3 * o, c->conv.p, sizeof(double) * 3 * m, hipMemcpyDeviceToHost, c->stream));
   }
+  if (n) sync(c);
 }
 template <class T>
 std::vector<T> download(phafd_hip_ctx *c, const T *d, size_t n) {
@@ -1783,8 +1813,8 @@ int phafd_hip_set_images(phafd_hip_ctx *c, const int *image) {
 }
 int phafd_hip_get_atoms(phafd_hip_ctx *c, double *xyz, double *uxyz, int *image) {
   return guard(c, [&] {
-    if (xyz) from_d4(download(c, c->x.p, c->nowned), xyz);
-    if (uxyz) from_d4(download(c, c->ux.p, c->nowned), uxyz);
+    if (xyz) download3(c, c->x.p, c->nowned, xyz);
+    if (uxyz) download3(c, c->ux.p, c->nowned, uxyz);
     if (image && c->nowned) {
       auto v = download(c, c->image.p, c->nowned);
       std::memcpy(image, v.data(), sizeof(int) * c->nowned);
@@ -1794,7 +1824,7 @@ int phafd_hip_get_atoms(phafd_hip_ctx *c, double *xyz, double *uxyz, int *image)
 }
 int phafd_hip_get_forces(phafd_hip_ctx *c, double *f) {
   return guard(c, [&] {
-    from_d4(download(c, c->F.p, c->nowned), f);
+    download3(c, c->F.p, c->nowned, f);
     return 0;
   });
 }
@@ -2029,7 +2059,7 @@ int phafd_hip_compute_pair(phafd_hip_ctx *c, int ipair, double *f) {
       }
     }
     reverse_comm(c);
-    from_d4(download(c, c->F.p, n), f);
+    download3(c, c->F.p, n, f);
     launch_copy4(n, c->cp_keep.p, c->F.p, c->stream);
     sync(c);
     return 0;
@@ -2545,7 +2575,7 @@ int phafd_hip_halflist(phafd_hip_ctx *c, int64_t cap, int *ilist, int *numneigh,
 int phafd_hip_gathered(phafd_hip_ctx *c, double *xyz, int *tag, int *label, int *owner) {
   return guard(c, [&] {
     const int ng = c->ngathered;
-    if (xyz) from_d4(download(c, c->gx.p, ng), xyz);
+    if (xyz) download3(c, c->gx.p, ng, xyz);
     auto own = download(c, c->gowner.p, ng);
     if (owner && ng) std::memcpy(owner, own.data(), sizeof(int) * ng);
     if (tag) for (int i = 0; i < ng; i++) tag[i] = c->h_tag[own[i]];
