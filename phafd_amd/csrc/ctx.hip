@@ -1116,7 +1116,7 @@ void phase_final_split(phafd_hip_ctx *c, bool atoms = true, bool next = false) {
     FixDef &f = *fp;
     if (f.kind == FixDef::CONJ && next) {
       const auto *nz = take_noise<R>(c, f);
-      fft_z_update_next(c->plan, F.muhat.p, F.phihat.p, F.ghat[0].p, F.ghat[2].p, nz, update_params(c, f),
+      fft_z_update_next(c->plan, F.muhat.p, F.phihat.p, F.ghat[0].p, F.ghat[1].p, F.ghat[2].p, nz, update_params(c, f),
                         origin_ptr(c), spec_const(c), c->stream, c->store_muhat);
     } else if (f.kind == FixDef::CONJ) {
       const auto *nz = take_noise<R>(c, f);

@@ -149,7 +149,7 @@ struct UpdateParams;
                     const double *origin, hipStream_t s, Slab sl = Slab(), bool store_mu = true);        \
   void fft_c2r_yx_batch(const FFTPlan &p, CT *const *in, RT *const *out, int batch, double divisor,      \
                         hipStream_t s);                                                                  \
-  void fft_z_update_next(const FFTPlan &p, CT *mu, CT *ph, CT *za, CT *zg, const CT *noise, UpdateParams u,  \
+  void fft_z_update_next(const FFTPlan &p, CT *mu, CT *ph, CT *za, CT *gy_k, CT *zg, const CT *noise, UpdateParams u,  \
                          const double *origin, SpecConst sc, hipStream_t s, bool store_mu);                \
   void fft_c2r_next(const FFTPlan &p, CT *za, CT *gy_k, CT *zg, RT *phi, RT *gx, RT *gy, RT *gz, SpecConst sc, \
                     hipStream_t s);                                                                         \
@@ -159,9 +159,10 @@ struct UpdateParams;
 // divides the output).  fft_c2r_batch: up to 4 spectra per launch.
 // fft_r2c_xy: the x and y passes of an r2c.  fft_grad_sep: the gradient of
 // phi by separable spectral derivatives (grids with fft_sep_grad_ok): gx from
-// one x-line kernel, gy from the y pass, gz from the z pass; ph receives
-// phihat; gy_k, gz_k are scratch spectra; equal in exact arithmetic to r2c,
-// grad multiply, three c2r / N.  fft_z_update: z pass of mu's r2c, the
+// one x-line kernel, gy and gz from phi's y and z lines and the Nyquist modes
+// of its transform (FP32 and small grids: from the y pass and the z pass); ph
+// receives phihat; gy_k, gz_k are scratch spectra; equal in exact arithmetic
+// to r2c, grad multiply, three c2r / N.  fft_z_update: z pass of mu's r2c, the
 // spectral update of phihat and the z pass of its c2r in one kernel (grids
 // with fft_fused_z_ok); finish with fft_c2r_yx_batch.  origin != nullptr
 // (FP32 form): the k = 0 mode is taken from the FP64 sum there.  store_mu
@@ -171,7 +172,8 @@ struct UpdateParams;
 // system): the update of a step that another step of the run follows, and
 // the c2r of phi together with the next step's gradient: phihat keeps N
 // times the updated spectrum (the next step's r2c of phi, up to rounding),
-// za and zg hold the z passes of phi and of its z gradient, gy_k is scratch;
+// za holds the z pass of phi, zg that of its z gradient where that is taken
+// through a spectrum, gy_k is scratch kept from the one call to the other;
 // phi and grad phi come out as the next step's start_of_step would make them.
 PHAFD_FFT_DECL(double, double2)
 PHAFD_FFT_DECL(float, float2)
