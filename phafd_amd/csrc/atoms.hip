@@ -704,86 +704,36 @@ __global__ __launch_bounds__(256) void k_ga_tile_rows(int nrow, int ntx, int nty
 __global__ void k_ga_pm_count(int nent, const int2 *__restrict__ ps, int *__restrict__ pcnt, int *__restrict__ rank) {
   GRID_STRIDE(e, nent) rank[e] = atomicAdd(&pcnt[ps[e].x], 1);
 }
-// per pair: its place in its point's segment, carrying (q, entry)
+// per pair: its q into its point's segment, in the order of the ranks
 __global__ void k_ga_pm_place(int nent, const int2 *__restrict__ ps, const int *__restrict__ rank,
-                              const int *__restrict__ amq, const int *__restrict__ poff, int *__restrict__ key,
-                              int *__restrict__ ent) {
+                              const int *__restrict__ amq, const int *__restrict__ poff, int *__restrict__ key) {
+  GRID_STRIDE(e, nent) key[poff[ps[e].x] + rank[e]] = amq[e];
+}
+// per pair: its slot = its point's start + the number of smaller q in the
+// segment (an atom lists a point once, so the keys of a segment differ).
+// Nothing is moved: a wave's 64 pairs are a few x runs of a few atoms, whose
+// points' segments lie together, so the keys come from a few cached lines and
+// the slots are written in the pairs' own order.  A thread per point that
+// sorted its segment (insertion, in memory past 8 keys) and scattered the
+// slots took 15.5 ms a build at 512^3 with 174M pairs, 251 us at 256^3 with
+// 4.5M, 374 us at 128^3 with 2.4M.
+__global__ __launch_bounds__(256) void k_ga_pm_rank(int nent, const int *__restrict__ poff,
+                                                    const int *__restrict__ amq, const int *__restrict__ key,
+                                                    int2 *__restrict__ ps) {
   GRID_STRIDE(e, nent) {
-    const int slot = poff[ps[e].x] + rank[e];
-    key[slot] = amq[e];
-    ent[slot] = e;
-  }
-}
-// each point's segment into ascending q, then ps[entry].y = its slot.
-// GM_U points per lane, 64 apart; segments of up to 8 are sorted in
-// registers (their loads issued together), longer ones in memory.
-constexpr int GM_U = 8;
-__global__ __launch_bounds__(256) void k_ga_pm_sort(size_t N, const int *__restrict__ poff, int *__restrict__ key,
-                                                    int *__restrict__ ent, int2 *__restrict__ ps) {
-  const size_t wbase = ((size_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64) * (64 * GM_U);
-  const int lane = threadIdx.x & 63;
-  int s[GM_U], n[GM_U];
-#pragma unroll
-  for (int u = 0; u < GM_U; u++) {
-    const size_t p = wbase + lane + 64 * u;
-    s[u] = p < N ? poff[p] : 0;
-    n[u] = p < N ? poff[p + 1] - s[u] : 0;
-  }
-#pragma unroll
-  for (int u = 0; u < GM_U; u++) {
-    const int a = s[u], m = n[u];
-    if (m == 0) continue;
-    if (m == 1) {
-      ps[ent[a]].y = a;
-    } else if (m == 2) {
-      const int k0 = key[a], k1 = key[a + 1], e0 = ent[a], e1 = ent[a + 1];
-      const bool sw = k0 > k1;
-      ps[sw ? e1 : e0].y = a;
-      ps[sw ? e0 : e1].y = a + 1;
-    } else if (m <= 8) {
-      int kk[8], ee[8];
-#pragma unroll
-      for (int i = 0; i < 8; i++) {
-        kk[i] = i < m ? key[a + i] : 0x7fffffff;
-        ee[i] = i < m ? ent[a + i] : 0;
-      }
-      // insertion sort over the fixed 8 (keys of a segment differ)
-#pragma unroll
-      for (int i = 1; i < 8; i++) {
-#pragma unroll
-        for (int j = i; j > 0; j--) {
-          const bool sw = kk[j - 1] > kk[j];
-          const int tk = sw ? kk[j - 1] : kk[j], te = sw ? ee[j - 1] : ee[j];
-          kk[j - 1] = sw ? kk[j] : kk[j - 1];
-          ee[j - 1] = sw ? ee[j] : ee[j - 1];
-          kk[j] = tk;
-          ee[j] = te;
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 8; i++) {
-        if (i < m) {
-          key[a + i] = kk[i];
-          ent[a + i] = ee[i];
-          ps[ee[i]].y = a + i;
-        }
-      }
-    } else {
-      for (int i = a + 1; i < a + m; i++) {
-        const int kv = key[i], ev = ent[i];
-        int j = i - 1;
-        while (j >= a && key[j] > kv) {
-          key[j + 1] = key[j];
-          ent[j + 1] = ent[j];
-          j--;
-        }
-        key[j + 1] = kv;
-        ent[j + 1] = ev;
-      }
-      for (int i = a; i < a + m; i++) ps[ent[i]].y = i;
+    const int p = ps[e].x, q = amq[e];
+    const int s = poff[p], t = poff[p + 1];
+    int n = 0, i = s;
+    for (; i + 4 <= t; i += 4) {
+      const int k0 = key[i], k1 = key[i + 1], k2 = key[i + 2], k3 = key[i + 3];
+      n += (k0 < q) + (k1 < q) + (k2 < q) + (k3 < q);
     }
+    for (; i < t; i++) n += key[i] < q;
+    ps[e].y = s + n;
   }
 }
+// points per lane of the mu sums
+constexpr int GM_U = 8;
 
 // The step's grid-atom pass, atom side: G lanes per atom (bin order q) take
 // its build pairs G at a time in ascending grid index, keep those in the pair
@@ -1916,14 +1866,12 @@ void launch_ga_pm_count(int nent, const int2 *ps, int *pcnt, int *rank, hipStrea
   hipLaunchKernelGGL(k_ga_pm_count, dim3(nblk(nent)), dim3(TPB), 0, s, nent, ps, pcnt, rank);
   HIPCHK(hipGetLastError());
 }
-void launch_ga_pm_place(int nent, int2 *ps, const int *rank, const int *amq, const int *poff, int *key, int *ent,
-                        size_t N, hipStream_t s) {
+void launch_ga_pm_place(int nent, int2 *ps, const int *rank, const int *amq, const int *poff, int *key,
+                        hipStream_t s) {
   if (nent <= 0) return;
-  hipLaunchKernelGGL(k_ga_pm_place, dim3(nblk(nent)), dim3(TPB), 0, s, nent, ps, rank, amq, poff, key, ent);
+  hipLaunchKernelGGL(k_ga_pm_place, dim3(nblk(nent)), dim3(TPB), 0, s, nent, ps, rank, amq, poff, key);
   HIPCHK(hipGetLastError());
-  const size_t per_block = 4 * 64 * GM_U;
-  hipLaunchKernelGGL(k_ga_pm_sort, dim3((unsigned)((N + per_block - 1) / per_block)), dim3(256), 0, s, N, poff, key,
-                     ent, ps);
+  hipLaunchKernelGGL(k_ga_pm_rank, dim3(nblk(nent)), dim3(TPB), 0, s, nent, poff, amq, key, ps);
   HIPCHK(hipGetLastError());
 }
 static int ilog2(int v) {

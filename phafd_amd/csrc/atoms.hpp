@@ -127,8 +127,8 @@ int64_t ga_tile_rows(const BinGeom &bg);
 void launch_ga_tile_rows(bool fill, const BinGeom &bg, const int *binstart, int *cnt, const int *off, int *perm,
                          hipStream_t s);
 void launch_ga_pm_count(int nent, const int2 *ps, int *pcnt, int *rank, hipStream_t s);
-void launch_ga_pm_place(int nent, int2 *ps, const int *rank, const int *amq, const int *poff, int *key, int *ent,
-                        size_t N, hipStream_t s);
+void launch_ga_pm_place(int nent, int2 *ps, const int *rank, const int *amq, const int *poff, int *key,
+                        hipStream_t s);
 // One grid-atom pair style (PairGridAtomGaussian / LJish / LJish/linear
 // compute) over the nent pairs of the last build.  launch_ga_force: gF(a) -= the
 // atom's terms in ascending grid index (FP32 form: Kahan-summed FP32 terms

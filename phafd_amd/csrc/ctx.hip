@@ -181,7 +181,7 @@ struct phafd_hip_ctx {
   // pass (NaN out of the cut)
   DBuf<int> ga_tcnt, ga_toff, ga_perm;   // wide couplings: the atoms in tile order
   bool ga_tiled = false;
-  DBuf<int> ga_acnt, ga_aoff, ga_amq, ga_rank, ga_pcnt, ga_poff, ga_key, ga_ent;
+  DBuf<int> ga_acnt, ga_aoff, ga_amq, ga_rank, ga_pcnt, ga_poff, ga_key;
   DBuf<int2> ga_ps;
   DBuf<double> ga_mterm;
   DBuf<float> ga_mterm32;
@@ -729,12 +729,10 @@ void build_ga_pairs(phafd_hip_ctx *c) {
   c->ga_poff.alloc(c->N + 2);
   c->ga_rank.alloc((size_t)nent + 1);
   c->ga_key.alloc((size_t)nent + 1);
-  c->ga_ent.alloc((size_t)nent + 1);
   fill_zero(c->ga_pcnt.p, sizeof(int) * c->N, c->stream);
   launch_ga_pm_count(nent, c->ga_ps.p, c->ga_pcnt.p, c->ga_rank.p, c->stream);
   scan_exclusive_i32(c->ga_pcnt.p, c->ga_poff.p, c->N, c->stream);
-  launch_ga_pm_place(nent, c->ga_ps.p, c->ga_rank.p, c->ga_amq.p, c->ga_poff.p, c->ga_key.p, c->ga_ent.p, c->N,
-                     c->stream);
+  launch_ga_pm_place(nent, c->ga_ps.p, c->ga_rank.p, c->ga_amq.p, c->ga_poff.p, c->ga_key.p, c->stream);
   if (c->fp32) c->ga_mterm32.alloc((size_t)nent + 1);
   else c->ga_mterm.alloc((size_t)nent + 1);
   c->ga_calls = c->ncalls;
