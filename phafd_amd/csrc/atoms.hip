@@ -732,9 +732,6 @@ __global__ __launch_bounds__(256) void k_ga_pm_rank(int nent, const int *__restr
     ps[e].y = s + n;
   }
 }
-// points per lane of the mu sums
-constexpr int GM_U = 8;
-
 // The step's grid-atom pass, atom side: G lanes per atom (bin order q) take
 // its build pairs G at a time in ascending grid index, keep those in the pair
 // cut now (the reference's test) and form their terms; the mu term of each
@@ -911,60 +908,65 @@ __global__ __launch_bounds__(256) void k_ga_force_multi(const GAMemberDev *__res
 
 // The step's grid-atom pass, grid side: mu(g) (first: from zero, else added
 // to) += the mu terms of its pairs, held in its segment in the reference's
-// list order, skipping the pairs out of the cut (NaN).  A wave takes
-// 64 * GM_U consecutive points, GM_U per lane 64 apart, and issues the loads
-// of its points (offsets, then up to four terms each) before using them.
-template <class R>
+// list order, skipping the pairs out of the cut (NaN).  A block takes 256 U
+// consecutive points, U per thread 256 apart, whose terms are one run of
+// mterm: the run comes to LDS GM_CH terms at a time (coalesced, all waves),
+// and each thread adds what a chunk holds of its points' segments.  Walking
+// the segments in global memory, a latency per term on lanes of unequal
+// lengths, the sums took (us a launch, before -> now): 66 -> 45 at 256^3 FP64
+// (5.3 TB/s, a copy's rate), 47 -> 37 FP32, 1055 -> 709 at 512^3 FP32 with
+// 174M pairs, 29 -> 15 at 128^3 with 2.4M, 5.5 -> 3.8 at 64^3.
+constexpr int GM_CH = 2048;   // terms staged at a time
+template <class R, int U>
 __device__ __forceinline__ void ga_list_mu_block(size_t blk, size_t N, R *__restrict__ mu,
                                                  const int *__restrict__ poff, const R *__restrict__ mterm,
                                                  int first) {
-  const size_t wbase = (blk * (blockDim.x / 64) + threadIdx.x / 64) * (64 * GM_U);
-  const int lane = threadIdx.x & 63;
-  int s[GM_U], n[GM_U];
-  R m[GM_U];
+  __shared__ R st[GM_CH];
+  const size_t p0 = blk * (256 * U);
+  const int tid = threadIdx.x;
+  int s[U], e[U];
+  MuAcc<R> acc[U];
 #pragma unroll
-  for (int u = 0; u < GM_U; u++) {
-    const size_t p = wbase + lane + 64 * u;
-    s[u] = p <= N ? poff[p] : 0;   // poff[N] is the total
-    m[u] = (first || p >= N) ? R(0) : mu[p];
+  for (int u = 0; u < U; u++) {
+    const size_t p = p0 + tid + 256 * u;
+    s[u] = p < N ? poff[p] : 0;   // poff[N] is the total
+    e[u] = p < N ? poff[p + 1] : 0;
+    acc[u].m = (first || p >= N) ? R(0) : mu[p];
   }
-  // a point's end is the next point's start: the next lane's, or for lane
-  // 63 the next row's lane 0 (one more load after the last row)
-  const size_t plast = wbase + 64 * GM_U;
-  const int tail = (lane == 63 && plast <= N) ? poff[plast] : 0;
+  const size_t p1 = p0 + 256 * U < N ? p0 + 256 * U : N;
+  const int b = poff[p0], t = poff[p1];
+  for (int c0 = b; c0 < t; c0 += GM_CH) {
+    const int c1 = t - c0 < GM_CH ? t : c0 + GM_CH;
 #pragma unroll
-  for (int u = 0; u < GM_U; u++) {
-    const int nxt = __shfl(s[u], (lane + 1) & 63, 64);
-    const int row0 = u + 1 < GM_U ? __shfl(s[u + 1 < GM_U ? u + 1 : u], 0, 64) : tail;
-    const size_t p = wbase + lane + 64 * u;
-    n[u] = p < N ? (lane == 63 ? row0 : nxt) - s[u] : 0;
-  }
-  R v0[GM_U];
+    for (int i = 0; i < GM_CH; i += 256)
+      if (c0 + i + tid < c1) st[i + tid] = mterm[c0 + i + tid];
+    __syncthreads();
 #pragma unroll
-  for (int u = 0; u < GM_U; u++) v0[u] = n[u] > 0 ? mterm[s[u]] : R(0);
-#pragma unroll
-  for (int u = 0; u < GM_U; u++) {
-    const size_t p = wbase + lane + 64 * u;
-    if (p >= N) continue;
-    MuAcc<R> acc;
-    acc.m = m[u];
-    if (n[u] > 0 && !isnan(v0[u])) acc.add(v0[u]);
-    for (int c = s[u] + 1; c < s[u] + n[u]; c++) {
-      const R x = mterm[c];
-      if (!isnan(x)) acc.add(x);
+    for (int u = 0; u < U; u++) {
+      const int hi = e[u] < c1 ? e[u] : c1;
+      for (; s[u] < hi; s[u]++) {
+        const R x = st[s[u] - c0];
+        if (!isnan(x)) acc[u].add(x);
+      }
     }
-    mu[p] = acc.get();
+    __syncthreads();
+  }
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const size_t p = p0 + tid + 256 * u;
+    if (p < N) mu[p] = acc[u].get();
   }
 }
-template <class R>
+template <class R, int U>
 __global__ __launch_bounds__(256) void k_ga_list_mu(size_t N, R *__restrict__ mu, const int *__restrict__ poff,
                                                     const R *__restrict__ mterm, int first) {
-  ga_list_mu_block<R>(blockIdx.x, N, mu, poff, mterm, first);
+  ga_list_mu_block<R, U>(blockIdx.x, N, mu, poff, mterm, first);
 }
 // every member's mu sums in one launch (blockIdx.y: the member; mu from zero)
+template <int U>
 __global__ __launch_bounds__(256) void k_ga_list_mu_multi(const GAMemberDev *__restrict__ d, size_t N) {
   const GAMemberDev &g = d[blockIdx.y];
-  ga_list_mu_block<double>(blockIdx.x, N, g.mu, g.poff, g.mterm, 1);
+  ga_list_mu_block<double, U>(blockIdx.x, N, g.mu, g.poff, g.mterm, 1);
 }
 
 // PairLJCut::compute, src/pair_lj_cut.cpp:46-119, gathered per atom: atom k
@@ -1889,6 +1891,9 @@ static int ilog2(int v) {
 // 108, not worth the order's build).  48 pairs per atom (reach 2.25, 128^3):
 // 16 lanes 4% less per step.  24 pairs, three rounds of 8 lanes, is between.
 bool ga_wide(int64_t ng, int64_t nent) { return nent >= 24 * ng; }
+// points per thread of the mu sums: four leave more loads in flight, but a
+// small grid needs its blocks to reach every CU (64^3: 256 blocks of four)
+int gm_points(size_t N) { return N >= (size_t)1 << 21 ? 4 : 1; }
 #define PHAFD_GA_DEF(RT)                                                                                        \
   void launch_ga_force(int ng, int64_t nent, const GridViewT<RT> &gv, const GAParams &ga, const double4 *gx,   \
                        const int *order, const int *perm, const int *aoff, const int2 *ps, RT *mterm, double4 *gF, \
@@ -1902,9 +1907,10 @@ bool ga_wide(int64_t ng, int64_t nent) { return nent >= 24 * ng; }
     HIPCHK(hipGetLastError());                                                                                \
   }                                                                                                           \
   void launch_ga_list_mu(size_t N, RT *mu, const int *poff, const RT *mterm, bool first, hipStream_t s) {     \
-    const size_t per_block = 4 * 64 * GM_U;                                                                   \
-    hipLaunchKernelGGL(k_ga_list_mu<RT>, dim3((unsigned)((N + per_block - 1) / per_block)), dim3(256), 0, s, N, \
-                       mu, poff, mterm, first ? 1 : 0);                                                       \
+    const int U = gm_points(N);                                                                               \
+    const auto k = U == 4 ? k_ga_list_mu<RT, 4> : k_ga_list_mu<RT, 1>;                                        \
+    hipLaunchKernelGGL(k, dim3((unsigned)((N + 256 * U - 1) / (256 * U))), dim3(256), 0, s, N, mu, poff,      \
+                       mterm, first ? 1 : 0);                                                                 \
     HIPCHK(hipGetLastError());                                                                                \
   }
 PHAFD_GA_DEF(double)
@@ -1992,9 +1998,9 @@ void launch_ga_force_multi(int nm, const GAMemberDev *d, const int *boff, int ni
 }
 void launch_ga_list_mu_multi(int nm, size_t N, const GAMemberDev *d, hipStream_t s) {
   if (nm <= 0) return;
-  const size_t per_block = 4 * 64 * GM_U;
-  hipLaunchKernelGGL(k_ga_list_mu_multi, dim3((unsigned)((N + per_block - 1) / per_block), nm), dim3(256), 0, s, d,
-                     N);
+  const int U = gm_points(N * nm);
+  hipLaunchKernelGGL(U == 4 ? k_ga_list_mu_multi<4> : k_ga_list_mu_multi<1>,
+                     dim3((unsigned)((N + 256 * U - 1) / (256 * U)), nm), dim3(256), 0, s, d, N);
   HIPCHK(hipGetLastError());
 }
 void launch_lj_multi(int nm, const LJMemberDev *d, const int *boff, int nitems, const MultiShape &sh,
