@@ -255,6 +255,75 @@ __global__ void k_reverse2(int ca, const int *sa, int fa, int cb, const int *sb,
   }
 }
 
+// Reverse comm in one launch.  An owned atom's images form a tree: at most
+// one along each dimension (disjoint swaps), each of which has its own along
+// the dimensions swapped after it.  slot[8 k + code] of the atom's list k =
+// idx[i] holds the image shifted along the dimensions of code (1 x, 2 y, 4
+// z), -1 where there is none; idx is -1 for the atoms without images.  The
+// sums nest as the swaps' folds do (x into every entry, then y, then z, then
+// the atom), so the forces are theirs bit for bit, without a launch per
+// dimension and without rewriting gF.  Needs every owned atom to be its own
+// LOCAL copy entry.
+// code of a ghost: the dimensions it is shifted along; its list is claimed
+// by whichever of the atom's ghosts comes first
+__device__ __forceinline__ int fold_code(const double4 &s) { return (s.x != 0) | (s.y != 0) << 1 | (s.z != 0) << 2; }
+__global__ void k_fold_init(int n, int nghost, int *__restrict__ idx, int *__restrict__ slot) {
+  GRID_STRIDE(i, n + 8 * (size_t)nghost) {
+    if (i < (size_t)n) idx[i] = -1;
+    else slot[i - n] = -1;
+  }
+}
+__global__ void k_fold_claim(int n, int nghost, const int *__restrict__ owner, int *__restrict__ idx) {
+  GRID_STRIDE(k, nghost) atomicCAS(&idx[owner[n + k]], -1, (int)k);
+}
+__global__ void k_fold_slots(int n, int nghost, const int *__restrict__ owner, const double4 *__restrict__ shift,
+                             const int *__restrict__ idx, int *__restrict__ slot) {
+  GRID_STRIDE(k, nghost) {
+    const int e = n + (int)k;
+    slot[8 * (size_t)idx[owner[e]] + fold_code(shift[e])] = e;
+  }
+}
+__device__ __forceinline__ void add3(double4 &a, const double4 &b) {
+  a.x += b.x;
+  a.y += b.y;
+  a.z += b.z;
+}
+// entry i of gF with its images folded in
+__device__ __forceinline__ double4 fold_atom(size_t i, const int *__restrict__ idx, const int *__restrict__ slot,
+                                             const double4 *__restrict__ gF) {
+  double4 b = gF[i];
+  const int k = idx[i];
+  if (k >= 0) {
+    int e[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) e[u] = slot[8 * (size_t)k + u];
+    double4 v[8];
+#pragma unroll
+    for (int u = 1; u < 8; u++)
+      if (e[u] >= 0) v[u] = gF[e[u]];
+    // x images into every entry, then y images, then z images
+    if (e[1] >= 0) add3(b, v[1]);
+    if (e[2] >= 0 && e[3] >= 0) add3(v[2], v[3]);
+    if (e[4] >= 0 && e[5] >= 0) add3(v[4], v[5]);
+    if (e[6] >= 0 && e[7] >= 0) add3(v[6], v[7]);
+    if (e[2] >= 0) add3(b, v[2]);
+    if (e[4] >= 0 && e[6] >= 0) add3(v[4], v[6]);
+    if (e[4] >= 0) add3(b, v[4]);
+  }
+  return b;
+}
+// F = init (null: zero) + the folded gF
+__global__ __launch_bounds__(256) void k_fold_tree(int n, const int *__restrict__ idx, const int *__restrict__ slot,
+                                                   const double4 *__restrict__ gF, const double4 *__restrict__ init,
+                                                   double4 *__restrict__ F, StepGate gate) {
+  if (gate_off(gate)) return;
+  GRID_STRIDE(i, n) {
+    double4 t = init ? init[i] : make_double4(0.0, 0.0, 0.0, 0.0);
+    add3(t, fold_atom(i, idx, slot, gF));
+    F[i] = t;
+  }
+}
+
 // ---------------------------------------------------------------- bins
 // NBin::coord2bin, src/nbin.cpp:61-94
 __device__ __forceinline__ int coord2bin(const BinGeom &b, double x, double y, double z) {
@@ -859,7 +928,7 @@ __device__ __forceinline__ void ga_force_atom(size_t q, bool on, const GridViewT
   if (ZI && on && sub == 3) Fa[3] = 0.0;
 }
 
-template <class R, int G>
+template <class R, int G, bool ZI>
 __global__ __launch_bounds__(256) void k_ga_force(int ng, GridViewT<R> gv, GAParams ga,
                                                   const double4 *__restrict__ gx, const int *__restrict__ order,
                                                   const int *__restrict__ perm, const int *__restrict__ aoff,
@@ -870,7 +939,7 @@ __global__ __launch_bounds__(256) void k_ga_force(int ng, GridViewT<R> gv, GAPar
   const size_t i = (size_t)xcd_block(blockIdx.x, gridDim.x) * (256 / G) + threadIdx.x / G;
   const bool on = i < (size_t)ng;
   const size_t q = perm && on ? (size_t)perm[i] : i;
-  ga_force_atom<R, false, G>(q, on, gv, ga, gx, order, aoff, ps, mterm, gF, sh[threadIdx.x / 64], esum,
+  ga_force_atom<R, ZI, G>(q, on, gv, ga, gx, order, aoff, ps, mterm, gF, sh[threadIdx.x / 64], esum,
                              energy != nullptr, lx, lxy);
   if (energy && esum != 0.0) atomicAdd(energy, esum);
 }
@@ -1099,6 +1168,21 @@ __global__ __launch_bounds__(256) void k_fold_multi(const FoldDev *__restrict__ 
     t.y += b.y;
     t.z += b.z;
     f.target[j] = t;
+  }
+}
+// the one-launch fold (k_fold_tree, F from zero) of every member: ca owned
+// atoms, lists sa (idx) and sb (slot)
+__global__ __launch_bounds__(256) void k_fold_tree_multi(const FoldDev *__restrict__ d, const int *__restrict__ boff,
+                                                         int nm) {
+  const int nitems = boff[nm];
+  for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
+    const int m = member_of(boff, nm, item);
+    const FoldDev &f = d[m];
+    const int i = (item - boff[m]) * blockDim.x + threadIdx.x;
+    if (i >= f.ca) continue;
+    double4 t = make_double4(0.0, 0.0, 0.0, 0.0);
+    add3(t, fold_atom(i, f.sa, f.sb, f.src));
+    f.target[i] = t;
   }
 }
 // the owned forces of every member set to zero (before a fold that adds)
@@ -1692,6 +1776,22 @@ void launch_reverse2(int ca, const int *sa, int fa, int cb, const int *sb, int f
   hipLaunchKernelGGL(k_reverse2, dim3(nblk(ca + cb)), dim3(TPB), 0, s, ca, sa, fa, cb, sb, fb, gF, gate);
   HIPCHK(hipGetLastError());
 }
+void launch_fold_lists(int n, int nghost, const GatheredView &g, int *idx, int *slot, hipStream_t s) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_fold_init, dim3(nblk(n + 8 * (size_t)nghost)), dim3(TPB), 0, s, n, nghost, idx, slot);
+  HIPCHK(hipGetLastError());
+  if (nghost <= 0) return;
+  hipLaunchKernelGGL(k_fold_claim, dim3(nblk(nghost)), dim3(TPB), 0, s, n, nghost, g.owner, idx);
+  HIPCHK(hipGetLastError());
+  hipLaunchKernelGGL(k_fold_slots, dim3(nblk(nghost)), dim3(TPB), 0, s, n, nghost, g.owner, g.shift, idx, slot);
+  HIPCHK(hipGetLastError());
+}
+void launch_fold_tree(int n, const int *idx, const int *slot, const double4 *gF, const double4 *init, double4 *F,
+                      hipStream_t s, StepGate gate) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_fold_tree, dim3(nblk(n)), dim3(TPB), 0, s, n, idx, slot, gF, init, F, gate);
+  HIPCHK(hipGetLastError());
+}
 void launch_atom2bin(int ng, const double4 *gx, const BinGeom &b, int *a2b, int *bincount, int *bad,
                      hipStream_t s) {
   if (ng <= 0) return;
@@ -1897,11 +1997,12 @@ int gm_points(size_t N) { return N >= (size_t)1 << 21 ? 4 : 1; }
 #define PHAFD_GA_DEF(RT)                                                                                        \
   void launch_ga_force(int ng, int64_t nent, const GridViewT<RT> &gv, const GAParams &ga, const double4 *gx,   \
                        const int *order, const int *perm, const int *aoff, const int2 *ps, RT *mterm, double4 *gF, \
-                       double *energy, hipStream_t s) {                                                       \
+                       double *energy, bool zero_init, hipStream_t s) {                                                       \
     if (ng <= 0) return;                                                                                      \
     const int lx = ilog2(gv.nx), lxy = lx + ilog2(gv.ny);                                                     \
     const int G = ga_wide(ng, nent) ? 16 : 8;                                                                 \
-    const auto k = G == 16 ? k_ga_force<RT, 16> : k_ga_force<RT, 8>;                                          \
+    const auto k = zero_init ? (G == 16 ? k_ga_force<RT, 16, true> : k_ga_force<RT, 8, true>)                 \
+                             : (G == 16 ? k_ga_force<RT, 16, false> : k_ga_force<RT, 8, false>);              \
     hipLaunchKernelGGL(k, dim3((unsigned)(((size_t)ng * G + 255) / 256)), dim3(256), 0, s, ng, gv, ga, gx,    \
                        order, perm, aoff, ps, mterm, gF, energy, lx, lxy);                                    \
     HIPCHK(hipGetLastError());                                                                                \
@@ -2016,6 +2117,12 @@ void launch_fold_multi(int nm, const FoldDev *d, const int *boff, int nitems, bo
   check_shape(sh);
   hipLaunchKernelGGL(k_fold_multi, dim3(multi_grid(nitems, sh.cap)), dim3(sh.threads), 0, s, d, boff, nm,
                      zero ? 1 : 0);
+  HIPCHK(hipGetLastError());
+}
+void launch_fold_tree_multi(int nm, const FoldDev *d, const int *boff, int nitems, const MultiShape &sh, hipStream_t s) {
+  if (nm <= 0 || nitems <= 0) return;
+  check_shape(sh);
+  hipLaunchKernelGGL(k_fold_tree_multi, dim3(multi_grid(nitems, sh.cap)), dim3(sh.threads), 0, s, d, boff, nm);
   HIPCHK(hipGetLastError());
 }
 void launch_fill_multi(int nm, const FoldDev *d, const int *boff, int nitems, const MultiShape &sh, hipStream_t s) {

@@ -82,6 +82,13 @@ void launch_reverse_init(int cnt, const int *send, int first, double4 *target, c
                          const double4 *gF, hipStream_t s, StepGate gate = StepGate());
 void launch_reverse2(int ca, const int *sa, int fa, int cb, const int *sb, int fb, double4 *gF, hipStream_t s,
                      StepGate gate = StepGate());
+// reverse comm as one fold per owned atom, where each owned atom is its own
+// LOCAL copy entry and the swaps of a dimension are disjoint: the image lists
+// of a build (idx: n, slot: 8 per ghost entry), and F = init (null: zero) +
+// the atom's gF with its images folded in, the sums of the swap by swap folds
+void launch_fold_lists(int n, int nghost, const GatheredView &g, int *idx, int *slot, hipStream_t s);
+void launch_fold_tree(int n, const int *idx, const int *slot, const double4 *gF, const double4 *init, double4 *F,
+                      hipStream_t s, StepGate gate = StepGate());
 void launch_atom2bin(int ng, const double4 *gx, const BinGeom &b, int *a2b, int *bincount, int *bad,
                      hipStream_t s);
 void launch_bin_place(int ng, const int *a2b, const int *binstart, int *cursor, int *binatoms, hipStream_t s);
@@ -133,13 +140,14 @@ void launch_ga_pm_place(int nent, int2 *ps, const int *rank, const int *amq, con
 // compute) over the nent pairs of the last build.  launch_ga_force: gF(a) -= the
 // atom's terms in ascending grid index (FP32 form: Kahan-summed FP32 terms
 // subtracted once); mterm[ps[entry].y] = the pair's mu term, NaN out of the
-// cut; energy (may be null) += the coupling energy.
+// cut; energy (may be null) += the coupling energy; zero_init: gF is written
+// from zero.
 // launch_ga_list_mu: mu(g) (first: from zero, else added to) += the terms
 // of its segment in order (ascending q, the reference's order).
 #define PHAFD_GA_DECL(RT)                                                                                       \
   void launch_ga_force(int ng, int64_t nent, const GridViewT<RT> &gv, const GAParams &ga, const double4 *gx,     \
                        const int *order, const int *perm, const int *aoff, const int2 *ps, RT *mterm,           \
-                       double4 *gF, double *energy, hipStream_t s);                                             \
+                       double4 *gF, double *energy, bool zero_init, hipStream_t s);                             \
   void launch_ga_list_mu(size_t N, RT *mu, const int *poff, const RT *mterm, bool first, hipStream_t s);
 PHAFD_GA_DECL(double)
 PHAFD_GA_DECL(float)
@@ -217,6 +225,8 @@ void launch_lj_multi(int nm, const LJMemberDev *d, const int *boff, int nitems, 
 void launch_fold_multi(int nm, const FoldDev *d, const int *boff, int nitems, bool zero, const MultiShape &sh,
                        hipStream_t s);
 // target[0 .. ca) = 0 of every member
+void launch_fold_tree_multi(int nm, const FoldDev *d, const int *boff, int nitems, const MultiShape &sh,
+                            hipStream_t s);
 void launch_fill_multi(int nm, const FoldDev *d, const int *boff, int nitems, const MultiShape &sh, hipStream_t s);
 // both half steps of the harmonic chains of every member (coff: chain offsets)
 void launch_chain_multi(int nm, const ChainMemberDev *d, const int *coff, int nchains, int maxlen, double dt,

@@ -148,6 +148,8 @@ struct phafd_hip_ctx {
   // gathered
   int ngathered = 0, nlocal = 0, nghost = 0, gcap = 0;
   DBuf<double4> gx, gshift, gF;
+  bool fold_tree = false;        // the last borders' ghosts fold in one launch (fold_idx, fold_slot)
+  DBuf<int> fold_idx, fold_slot;
   DBuf<int> gowner, glabel;
   DBuf<int> tmp_flag, tmp_pos, tmp_cat, tmp_part;
   std::vector<SwapDev> swaps;
@@ -416,6 +418,14 @@ void borders(phafd_hip_ctx *c) {
     iswap += 2;
   }
   c->nghost = c->ngathered - c->nlocal;
+  // the fold lists, where one pass can fold the ghost forces
+  c->fold_tree = z.count == n && c->nlocal == n;
+  for (size_t k = 1; k < c->swaps.size(); k += 2) c->fold_tree = c->fold_tree && c->swaps[k + 1].disjoint_pair;
+  if (c->fold_tree) {
+    c->fold_idx.alloc((size_t)n + 1);
+    c->fold_slot.alloc(8 * (size_t)c->nghost + 1);
+    launch_fold_lists(n, c->nghost, c->gview(), c->fold_idx.p, c->fold_slot.p, c->stream);
+  }
 }
 
 void forward_comm(phafd_hip_ctx *c, StepGate gate = StepGate()) {
@@ -428,6 +438,10 @@ void forward_comm(phafd_hip_ctx *c, StepGate gate = StepGate()) {
 void reverse_comm_from(phafd_hip_ctx *c, const double4 *init, StepGate gate = StepGate());
 
 void reverse_comm(phafd_hip_ctx *c) {
+  if (c->fold_tree) {
+    launch_fold_tree(c->nowned, c->fold_idx.p, c->fold_slot.p, c->gF.p, c->F.p, c->F.p, c->stream);
+    return;
+  }
   for (int iswap = (int)c->swaps.size() - 1; iswap >= 1; iswap--) {
     SwapDev &w = c->swaps[iswap];
     if (w.disjoint_pair) {   // the dimension's two swaps in one launch (same sums)
@@ -445,6 +459,10 @@ void reverse_comm(phafd_hip_ctx *c) {
 bool reverse_from_one_pass(const phafd_hip_ctx *c) { return c->swaps[0].count == c->nowned; }
 void reverse_comm_from(phafd_hip_ctx *c, const double4 *init, StepGate gate) {
   SwapDev &z = c->swaps[0];
+  if (c->fold_tree) {
+    launch_fold_tree(c->nowned, c->fold_idx.p, c->fold_slot.p, c->gF.p, init, c->F.p, c->stream, gate);
+    return;
+  }
   if (!reverse_from_one_pass(c)) {
     if (gate.stop) throw std::logic_error("gated fold needs the one-pass copy swap");
     launch_copy4(c->nowned, init, c->F.p, c->stream);
@@ -948,11 +966,12 @@ void phase_neigh(phafd_hip_ctx *c) {
 // of the terms in the reference's list order (or, with the eager option,
 // the walk of the stored NPairGridBin list; the two are bit-identical).
 // first: mu has not been zeroed this step; the pass writes every point.
+// zero_init: gF neither, the pass writes every entry.
 template <class R> DBuf<R> &ga_mterm(phafd_hip_ctx *c);
 template <> DBuf<double> &ga_mterm<double>(phafd_hip_ctx *c) { return c->ga_mterm; }
 template <> DBuf<float> &ga_mterm<float>(phafd_hip_ctx *c) { return c->ga_mterm32; }
 template <class R>
-void grid_atom_pass(phafd_hip_ctx *c, PairDef &p, double *energy, bool first) {
+void grid_atom_pass(phafd_hip_ctx *c, PairDef &p, double *energy, bool first, bool zero_init = false) {
   FieldSet<R> &Fs = c->fields<R>();
   const GridViewT<R> gvr = c->gridview<R>();
   GAParams ga = ga_params(p);
@@ -963,7 +982,7 @@ void grid_atom_pass(phafd_hip_ctx *c, PairDef &p, double *energy, bool first) {
   // gathered atom's position read and force written
   probe_begin(K_GA_FORCE, c->stream);
   launch_ga_force(c->ngathered, c->ga_nent, gvr, ga, c->gx.p, c->binatoms.p, c->ga_tiled ? c->ga_perm.p : nullptr,
-                  c->ga_aoff.p, c->ga_ps.p, mt.p, c->gF.p, energy, c->stream);
+                  c->ga_aoff.p, c->ga_ps.p, mt.p, c->gF.p, energy, zero_init, c->stream);
   probe_end(K_GA_FORCE, c->stream, 4.0 * sizeof(R) * c->N + 64.0 * c->ngathered);
   probe_begin(K_GA_DEPOSIT, c->stream);
   if (!(c->eager_gridlist && c->grid_built)) {
@@ -990,27 +1009,32 @@ void phase_pair(phafd_hip_ctx *c, double *energy_ga = nullptr, double *energy_lj
     fill_zero(c->fp32 ? (void *)c->fs.mu.p : (void *)c->fd.mu.p, c->real_bytes() * c->N, c->stream);
     mu_pending = false;
   }
-  launch_fill_d4(c->ngathered, c->gF.p, c->stream);
-  launch_fill_d4(c->nowned, c->F.p, c->stream);
-  if (!c->neigh_set || !c->lists_valid) return;
+  // gF from zero: by the first style's pass; F from zero: by the fold
+  const bool lists = c->neigh_set && c->lists_valid;
+  bool gf_pending = lists && !c->pairs.empty();
+  if (!gf_pending) launch_fill_d4(c->ngathered, c->gF.p, c->stream);
+  if (!lists || !c->fold_tree) launch_fill_d4(c->nowned, c->F.p, c->stream);
+  if (!lists) return;
   for (auto &pp : c->pairs) {
     PairDef &p = *pp;
     if (p.style == 2) {
       LJParams lj{p.lj1, p.lj2, p.ljcutsq};
       probe_begin(K_LJ, c->stream);
       launch_lj_force(c->ngathered, lj, c->gx.p, c->h_rowof.p, c->h_off.p, c->h_neigh.p, c->t_off.p,
-                      c->t_pair.p, c->t_i.p, c->nowned, c->gF.p, energy_lj, c->stream);
+                      c->t_pair.p, c->t_i.p, c->nowned, c->gF.p, energy_lj, c->stream, gf_pending);
       probe_end(K_LJ, c->stream, 64.0 * c->ngathered + 4.0 * c->h_nent);
     } else if (p.style == 4) {
       launch_harmonic_force(c->ngathered, HarmParams{p.hk, p.hcut}, c->gx.p, c->h_rowof.p, c->h_off.p, c->h_neigh.p,
-                            c->t_off.p, c->t_pair.p, c->t_i.p, c->nowned, c->gF.p, c->stream);
+                            c->t_off.p, c->t_pair.p, c->t_i.p, c->nowned, c->gF.p, c->stream, gf_pending);
     } else {
-      if (c->fp32) grid_atom_pass<float>(c, p, energy_ga, mu_pending);
-      else grid_atom_pass<double>(c, p, energy_ga, mu_pending);
+      if (c->fp32) grid_atom_pass<float>(c, p, energy_ga, mu_pending, gf_pending);
+      else grid_atom_pass<double>(c, p, energy_ga, mu_pending, gf_pending);
       mu_pending = false;
     }
+    gf_pending = false;
   }
-  reverse_comm(c);
+  if (c->fold_tree) reverse_comm_from(c, nullptr);
+  else reverse_comm(c);
 }
 
 // second: the final_integrate half (FixAtomDrag and the harmonic chains do
@@ -3117,7 +3141,7 @@ void batch_pair_fused(phafd_hip_batch *b, bool with_chains) {
   for (auto &m : b->members) P.onepass = P.onepass && reverse_from_one_pass(m.get());
   std::vector<GAMemberDev> ga(nm);
   std::vector<LJMemberDev> lj(nm);
-  std::vector<FoldDev> fold((size_t)(P.nlev + 1) * nm);   // levels, then the fill of F
+  std::vector<FoldDev> fold((size_t)(P.nlev + 1) * nm);   // levels, then the fill of F or the one-launch fold
   std::vector<ChainMemberDev> ch(nm);
   const int stride = nm + 1;
   P.ints.assign((size_t)stride * (P.nlev + 4), 0);
@@ -3153,8 +3177,8 @@ void batch_pair_fused(phafd_hip_batch *b, bool with_chains) {
       int *bo = boff_fold + (size_t)L * stride;
       bo[i + 1] = bo[i] + (f.ca + f.cb + T - 1) / T;
     }
-    FoldDev &fz = fold[(size_t)P.nlev * nm + i];   // the fill of F
-    fz = FoldDev{c->nowned, 0, 0, 0, nullptr, nullptr, c->F.p, nullptr};
+    FoldDev &fz = fold[(size_t)P.nlev * nm + i];
+    fz = FoldDev{c->nowned, 0, 0, 0, c->fold_idx.p, c->fold_slot.p, c->F.p, c->gF.p};
     int *bz = boff_fold + (size_t)P.nlev * stride;
     bz[i + 1] = bz[i] + (c->nowned + T - 1) / T;
     if (P.chains) {
@@ -3207,7 +3231,12 @@ void batch_pair_fused(phafd_hip_batch *b, bool with_chains) {
   probe_end(K_GA_FORCE, b->stream, 4.0 * sizeof(double) * b->N * nm + 64.0 * ng_all);
   launch_ga_list_mu_multi(nm, b->N, dga, b->stream);
   if (P.lj) launch_lj_multi(nm, dlj, dboff_ga, P.items_ga, b->shape, b->stream);
-  for (int L = 0; L < P.nlev; L++) {
+  bool tree = true;
+  for (auto &m : b->members) tree = tree && m->fold_tree;
+  if (tree)
+    launch_fold_tree_multi(nm, dfold + (size_t)P.nlev * nm, dboff_fold + (size_t)P.nlev * stride,
+                           boff_fold[(size_t)P.nlev * stride + nm], b->shape, b->stream);
+  for (int L = 0; !tree && L < P.nlev; L++) {
     const bool copy_swap = levels[L].first == 0;
     if (copy_swap && !P.onepass)
       launch_fill_multi(nm, dfold + (size_t)P.nlev * nm, dboff_fold + (size_t)P.nlev * stride,
