@@ -91,18 +91,19 @@ __global__ void k_unmap(int n, const double4 *x, double4 *ux, const int *image, 
 // clear != nullptr: block 0 also zeroes *clear (the flag of the step after)
 // gate.stop non-null: a speculative window's step; a decision records its
 // step in *gate.stop (the first one wins)
+__device__ __forceinline__ int decide_atom(const double4 &a, const double4 &h, double triggersq) {
+  const double d0 = a.x - h.x, d1 = a.y - h.y, d2 = a.z - h.z;
+  const double rsq = d0 * d0 + d1 * d1 + d2 * d2;
+  int f = rsq > triggersq ? 1 : 0;
+  if (!isfinite(a.x) || !isfinite(a.y) || !isfinite(a.z)) f |= 2;   // reported as an error
+  return f;
+}
 __global__ void k_decide(int n, const double4 *x, const double4 *xh, double triggersq, int *flag, int *clear,
                          StepGate gate) {
   if (gate_off(gate)) return;
   if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
   int f = 0;
-  GRID_STRIDE(i, n) {
-    const double4 a = x[i], h = xh[i];
-    const double d0 = a.x - h.x, d1 = a.y - h.y, d2 = a.z - h.z;
-    const double rsq = d0 * d0 + d1 * d1 + d2 * d2;
-    if (rsq > triggersq) f |= 1;
-    if (!isfinite(a.x) || !isfinite(a.y) || !isfinite(a.z)) f |= 2;   // reported as an error
-  }
+  GRID_STRIDE(i, n) f |= decide_atom(x[i], xh[i], triggersq);
   if (f) {
     atomicOr(flag, f);
     if (gate.stop) atomicCAS(gate.stop, 0, gate.step);
@@ -189,20 +190,34 @@ __global__ void k_img_scatter(int nscan, const int *flag, const int *pos, int di
 // swaps add 0.0, which is exact), so one pass reproduces the swap sequence.
 // Local copies (label 1) carry a zero shift, so only ghosts read theirs; the
 // type in .w is the owner's (as the border swaps set it).
+__device__ __forceinline__ void forward_entry(size_t i, const double4 *x, const int *type, const GatheredView &g) {
+  const int o = g.owner[i];
+  const double4 p = x[o];
+  double sx = 0.0, sy = 0.0, sz = 0.0;
+  if (g.label[i] != 1) {
+    const double4 s = g.shift[i];
+    sx = s.x;
+    sy = s.y;
+    sz = s.z;
+  }
+  g.x[i] = make_double4(p.x + sx, p.y + sy, p.z + sz, (double)type[o]);
+}
 __global__ void k_forward(int ng, const double4 *x, const int *type, GatheredView g, StepGate gate) {
   if (gate_off(gate)) return;
-  GRID_STRIDE(i, ng) {
-    const int o = g.owner[i];
-    const double4 p = x[o];
-    double sx = 0.0, sy = 0.0, sz = 0.0;
-    if (g.label[i] != 1) {
-      const double4 s = g.shift[i];
-      sx = s.x;
-      sy = s.y;
-      sz = s.z;
-    }
-    g.x[i] = make_double4(p.x + sx, p.y + sy, p.z + sz, (double)type[o]);
+  GRID_STRIDE(i, ng) forward_entry(i, x, type, g);
+}
+// A step's rebuild decision (k_decide) and the next step's forward comm in one
+// launch: both read the positions the step has just moved.  Where the decision
+// is to rebuild, the build writes the gathered atoms anew.
+__global__ void k_decide_forward(int n, int ng, const double4 *x, const double4 *xh, double triggersq, int *flag,
+                                 int *clear, const int *type, GatheredView g) {
+  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
+  int f = 0;
+  GRID_STRIDE(i, n > ng ? n : ng) {
+    if (i < (size_t)n) f |= decide_atom(x[i], xh[i], triggersq);
+    if (i < (size_t)ng) forward_entry(i, x, type, g);
   }
+  if (f) atomicOr(flag, f);
 }
 
 // CommBrick::reverse_comm for one swap, src/comm_brick.cpp:228-258 +
@@ -1751,6 +1766,16 @@ void launch_img_scatter(int nscan, const int *flag, const int *pos, int dim, dou
                         int *send, GatheredView g, hipStream_t s) {
   if (nscan <= 0) return;
   hipLaunchKernelGGL(k_img_scatter, dim3(nblk(nscan)), dim3(TPB), 0, s, nscan, flag, pos, dim, shift, first, send, g);
+  HIPCHK(hipGetLastError());
+}
+void launch_decide_forward(int n, int ng, const double4 *x, const double4 *xh, double triggersq, int *flag, int *clear,
+                           const int *type, GatheredView g, hipStream_t s) {
+  if (n <= 0) {
+    launch_fill_i32(1, clear, 0, s);
+    return;
+  }
+  hipLaunchKernelGGL(k_decide_forward, dim3(nblk(std::max(n, ng))), dim3(TPB), 0, s, n, ng, x, xh, triggersq, flag,
+                     clear, type, g);
   HIPCHK(hipGetLastError());
 }
 void launch_forward(int ng, const double4 *x, const int *type, GatheredView g, hipStream_t s, StepGate gate) {

@@ -194,6 +194,7 @@ struct phafd_hip_ctx {
   DBuf<int> t_cnt, t_off, t_cur, t_pair, t_i;
   bool lists_valid = false;
   int pending_decision = -1;   // rebuild decision prefetched at the end of the last step
+  bool gx_ahead = false;       // inside a run: the gathered positions are already the next step's
   bool store_muhat = true;     // the fused z update writes muhat (false inside a run but its last step)
   // in_fourier: the last step of a run copies ft_phi (before the update) and
   // ft_chempot (K layout, FP64) for compute complex / fix grid/ave
@@ -778,8 +779,15 @@ int decide_slot(const phafd_hip_ctx *c) { return 4 * (int)(c->timestep & 1); }
 void clear_decide_slot(phafd_hip_ctx *c, int64_t step) {
   launch_fill_i32(1, c->flags.p + 4 * (int)(step & 1), 0, c->stream);
 }
-void enqueue_decide(phafd_hip_ctx *c) {
+// forward: with the next step's forward comm (gx_ahead)
+void enqueue_decide(phafd_hip_ctx *c, bool forward = false) {
   const int sl = decide_slot(c);
+  if (forward) {
+    launch_decide_forward(c->nowned, c->ngathered, c->x.p, c->xhold.p, c->triggersq, c->flags.p + sl,
+                          c->flags.p + (4 - sl), c->type.p, c->gview(), c->stream);
+    c->gx_ahead = true;
+    return;
+  }
   launch_decide(c->nowned, c->x.p, c->xhold.p, c->triggersq, c->flags.p + sl, c->flags.p + (4 - sl), c->stream);
 }
 // the step's flags to h_flags[8..15], read after the step's synchronise
@@ -955,9 +963,10 @@ void phase_neigh(phafd_hip_ctx *c) {
     launch_pbc(c->nowned, c->x.p, c->ux.p, c->image.p, c->box(), c->stream);
     borders(c);
     neighbor_build(c);
-  } else {
+  } else if (!c->gx_ahead) {
     forward_comm(c);
   }
+  c->gx_ahead = false;
 }
 
 // One grid-atom pair style (PairGridAtomGaussian / PairGridAtomLJish
@@ -1150,11 +1159,11 @@ void phase_final_split(phafd_hip_ctx *c, bool atoms = true, bool next = false) {
   }
 }
 template <class R>
-void phase_postfinal_split(phafd_hip_ctx *c, bool next = false) {
+void phase_postfinal_split(phafd_hip_ctx *c, bool next = false, int *h_phi0 = nullptr) {
   FieldSet<R> &F = c->fields<R>();
   if (next) {
     fft_c2r_next(c->plan, F.ghat[0].p, F.ghat[1].p, F.ghat[2].p, F.phi.p, F.grad[0].p, F.grad[1].p, F.grad[2].p,
-                 spec_const(c), c->stream);
+                 spec_const(c), reinterpret_cast<R *>(h_phi0 ? h_phi0 : c->h_flags + 2), c->stream);
     c->grad_ready = true;
     return;
   }
@@ -1260,6 +1269,14 @@ template <class R>
 void run_steps_pipelined(phafd_hip_ctx *c, int nsteps, bool fused, bool zsplit, bool next_ok, FHPreT<R> &pre,
                          FixDef *fc) {
   auto phi0_slot = [&](int set) { return c->h_flags + (set ? 16 : 2); };
+  // The flags come with the r2c of mu where it applies Flory-Huggins, and a
+  // followed step's phi(0,0,0) with the c2r that makes it: a launch and an
+  // event less each than a copy of their own.
+  hipEvent_t ended[2];   // the last event of each parity's step
+  struct Ahead {         // an exception leaves the gathered positions as they are
+    bool &f;
+    ~Ahead() { f = false; }
+  } ahead{c->gx_ahead};
   // the timers and the NaN check of a completed step
   auto finish = [&](int set, int64_t step) {
     hipEvent_t *E = c->evp[set];
@@ -1269,7 +1286,7 @@ void run_steps_pipelined(phafd_hip_ctx *c, int nsteps, bool fused, bool zsplit, 
       c->tacc[k] += ms;
     }
     float tot = 0;
-    HIPCHK(hipEventElapsedTime(&tot, E[0], E[8]));
+    HIPCHK(hipEventElapsedTime(&tot, E[0], ended[set]));
     c->tacc[7] += tot;
     R phi0;
     std::memcpy(&phi0, phi0_slot(set), sizeof(R));
@@ -1301,10 +1318,15 @@ void run_steps_pipelined(phafd_hip_ctx *c, int nsteps, bool fused, bool zsplit, 
     else phase_initial(c);
     HIPCHK(hipEventRecord(E[4], c->stream));
     // next step's rebuild decision (Neighbor::decide): the atoms are final
-    if (c->neigh_set) enqueue_decide(c);
-    enqueue_flags_readback(c);
-    HIPCHK(hipEventRecord(E[9], c->stream));
-    if (!fused) phase_postforce_t<R>(c);
+    if (c->neigh_set) enqueue_decide(c, !last && c->lists_valid);
+    if (fused) {
+      pre.flags = c->flags.p;
+      pre.h_flags = c->h_flags + 8;
+    } else {
+      enqueue_flags_readback(c);
+      HIPCHK(hipEventRecord(E[9], c->stream));
+      phase_postforce_t<R>(c);
+    }
     if (zsplit) phase_prefinal_split<R>(c, fused ? &pre : nullptr);
     else phase_prefinal_t<R>(c, fused ? &pre : nullptr);
     HIPCHK(hipEventRecord(E[5], c->stream));
@@ -1314,7 +1336,7 @@ void run_steps_pipelined(phafd_hip_ctx *c, int nsteps, bool fused, bool zsplit, 
     if (zsplit) phase_final_split<R>(c, !fc, next);
     else phase_final_t<R>(c, !fc);
     HIPCHK(hipEventRecord(E[6], c->stream));
-    if (zsplit) phase_postfinal_split<R>(c, next);
+    if (zsplit) phase_postfinal_split<R>(c, next, phi0_slot(set));
     else phase_postfinal_t<R>(c);
     if (capture) {   // ft_chempot: the last step of a run stores the complete muhat
       capture_spectrum(c, 1, c->fields<R>().muhat.p);
@@ -1322,10 +1344,14 @@ void run_steps_pipelined(phafd_hip_ctx *c, int nsteps, bool fused, bool zsplit, 
     }
     HIPCHK(hipEventRecord(E[7], c->stream));
     // NaN check of phi(0,0,0) (src/integrate.cpp:190-201)
-    HIPCHK(hipMemcpyAsync(phi0_slot(set), c->fields<R>().phi.p, sizeof(R), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipEventRecord(E[8], c->stream));
+    ended[set] = E[7];
+    if (!next) {
+      HIPCHK(hipMemcpyAsync(phi0_slot(set), c->fields<R>().phi.p, sizeof(R), hipMemcpyDeviceToHost, c->stream));
+      HIPCHK(hipEventRecord(E[8], c->stream));
+      ended[set] = E[8];
+    }
     // this step's flags (mid-step); the previous step is complete by now
-    HIPCHK(hipEventSynchronize(E[9]));
+    HIPCHK(hipEventSynchronize(fused ? E[5] : E[9]));
     if (prev_step >= 0) finish(set ^ 1, prev_step);
     try {
       check_step_flags(c, step);

@@ -168,8 +168,8 @@ __host__ __device__ __forceinline__ C mk2(R x, R y) { return make_float2(x, y); 
     NS::fft_z_update_next_p(p, mu, ph, za, gy_k, zg, noise, u, origin, sc, s, store_mu);                           \
   }                                                                                                          \
   void fft_c2r_next(const FFTPlan &p, CT *za, CT *gy_k, CT *zg, RT *phi, RT *gx, RT *gy, RT *gz, SpecConst sc, \
-                    hipStream_t s) {                                                                         \
-    NS::fft_c2r_next_p(p, za, gy_k, zg, phi, gx, gy, gz, sc, s);                                             \
+                    RT *h_phi0, hipStream_t s) {                                                             \
+    NS::fft_c2r_next_p(p, za, gy_k, zg, phi, gx, gy, gz, sc, h_phi0, s);                                             \
   }                                                                                                          \
   void spec_k_to_canon(const FFTPlan &p, const CT *k, CT *canon, hipStream_t s) {                           \
     NS::spec_k_to_canon_p(p, k, canon, s);                                                                     \

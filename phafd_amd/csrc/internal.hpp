@@ -128,6 +128,9 @@ struct FHPreT {
   double tv = 1, chi = 1;     // temp/volFH, chi
   unsigned long long *counters = nullptr;   // [nless, ngreat] (per replica in a slab)
   const double *chi_b = nullptr;            // per-replica chi in a slab, or nullptr
+  // eight flags the launch copies to (device-visible) host memory, or null
+  const int *flags = nullptr;
+  int *h_flags = nullptr;
 };
 using FHPre = FHPreT<double>;
 
@@ -152,7 +155,7 @@ struct UpdateParams;
   void fft_z_update_next(const FFTPlan &p, CT *mu, CT *ph, CT *za, CT *gy_k, CT *zg, const CT *noise, UpdateParams u,  \
                          const double *origin, SpecConst sc, hipStream_t s, bool store_mu);                \
   void fft_c2r_next(const FFTPlan &p, CT *za, CT *gy_k, CT *zg, RT *phi, RT *gx, RT *gy, RT *gz, SpecConst sc, \
-                    hipStream_t s);                                                                         \
+                    RT *h_phi0, hipStream_t s);                                                                         \
   void spec_k_to_canon(const FFTPlan &p, const CT *k, CT *canon, hipStream_t s);                         \
   void spec_canon_to_k(const FFTPlan &p, const CT *canon, CT *k, hipStream_t s);
 // fft_r2c / fft_c2r: whole transforms (c2r destroys `in`; divisor != 0
@@ -174,7 +177,8 @@ struct UpdateParams;
 // times the updated spectrum (the next step's r2c of phi, up to rounding),
 // za holds the z pass of phi, zg that of its z gradient where that is taken
 // through a spectrum, gy_k is scratch kept from the one call to the other;
-// phi and grad phi come out as the next step's start_of_step would make them.
+// phi and grad phi come out as the next step's start_of_step would make them;
+// h_phi0 (device-visible host memory) receives phi(0, 0, 0).
 PHAFD_FFT_DECL(double, double2)
 PHAFD_FFT_DECL(float, float2)
 #undef PHAFD_FFT_DECL
