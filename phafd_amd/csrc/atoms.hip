@@ -1214,14 +1214,16 @@ __global__ __launch_bounds__(256) void k_fill_multi(const FoldDev *__restrict__ 
 // ---------------------------------------------------------- integrators
 // FixAtomDrag half step, src/fixatom_drag.cpp:43-66
 __global__ void k_drag(int n, const int *members, double4 *x, const double4 *F, double drag,
-                       double dt) {
+                       double dt, int halves) {
   GRID_STRIDE(q, n) {
     const int j = members[q];
     double4 p = x[j];
     const double4 f = F[j];
-    p.x += drag * f.x * dt * 0.5;
-    p.y += drag * f.y * dt * 0.5;
-    p.z += drag * f.z * dt * 0.5;
+    for (int h = 0; h < halves; h++) {
+      p.x += drag * f.x * dt * 0.5;
+      p.y += drag * f.y * dt * 0.5;
+      p.z += drag * f.z * dt * 0.5;
+    }
     x[j] = p;
   }
 }
@@ -2059,9 +2061,9 @@ void launch_harmonic_force(int ng, const HarmParams &h, const double4 *gx, const
   HIPCHK(hipGetLastError());
 }
 void launch_drag(int n, const int *members, double4 *x, const double4 *F, double drag, double dt,
-                 hipStream_t s) {
+                 hipStream_t s, int halves) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_drag, dim3(nblk(n)), dim3(TPB), 0, s, n, members, x, F, drag, dt);
+  hipLaunchKernelGGL(k_drag, dim3(nblk(n)), dim3(TPB), 0, s, n, members, x, F, drag, dt, halves);
   HIPCHK(hipGetLastError());
 }
 void launch_chain_step(int nchains, int maxlen, const int *chs, const int *che, const double4 *F, double4 *ux,

@@ -166,7 +166,7 @@ void launch_harmonic_force(int ng, const HarmParams &h, const double4 *gx, const
                            const int *hneigh, const int *toff, const int *tpair, const int *ti, int nowned,
                            double4 *gF, hipStream_t s, bool zero_init = false, StepGate gate = StepGate());
 void launch_drag(int n, const int *members, double4 *x, const double4 *F, double drag, double dt,
-                 hipStream_t s);
+                 hipStream_t s, int halves = 1);
 // halves (1 or 2) half steps of the chains (contiguous atom ranges
 // [chs[c], che[c]), at most maxlen beads, halves * maxlen * 32 bytes of LDS
 // per block); 2: both halves of a timestep, with the same F

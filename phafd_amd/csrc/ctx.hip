@@ -215,7 +215,6 @@ struct phafd_hip_ctx {
   bool setup_done = false;
   // timers
   hipEvent_t ev[9] = {};
-  hipEvent_t ev_pre[2] = {};   // a start_of_step enqueued ahead of the last read-back
   hipEvent_t evp[2][10] = {};  // pipelined steps: hook events 0-8 and the flags' read-back, per step parity
   double tacc[8] = {0};
   bool fuse_fh = true;
@@ -1074,6 +1073,27 @@ void phase_initial(phafd_hip_ctx *c) {
   for (auto &f : c->fixes) integrate_half(c, *f);
 }
 
+// Both half steps of every atom integrator, at initial_integrate.  F is made
+// once per step by the pair pass and the hooks between initial_integrate and
+// final_integrate work on the fields only, so the positions are those of the
+// halves in their places; the first halves of all fixes come before the
+// second ones, as there.
+void integrate_step(phafd_hip_ctx *c) {
+  FixDef *one = nullptr;
+  int n = 0;
+  for (auto &f : c->fixes)
+    if (f->kind == FixDef::DRAG || f->kind == FixDef::CHAIN || f->kind == FixDef::SEMIFLEX) {
+      one = f.get();
+      n++;
+    }
+  if (n == 1 && one->kind == FixDef::DRAG) {   // nothing between its halves
+    launch_drag(one->nmem, one->members.p, c->x.p, c->F.p, one->drag, c->dt, c->stream, 2);
+    return;
+  }
+  phase_initial(c);
+  for (auto &f : c->fixes) integrate_half(c, *f, true);
+}
+
 // The chain fix when it is the only atom integrator (and its chains fit two
 // LDS buffers of 32 KB): then both half steps of a timestep run as one
 // launch at initial_integrate.  F is computed once per step by the pair pass
@@ -1315,7 +1335,7 @@ void run_steps_pipelined(phafd_hip_ctx *c, int nsteps, bool fused, bool zsplit, 
     phase_pair(c);
     HIPCHK(hipEventRecord(E[3], c->stream));
     if (fc) integrate_both_halves(c, *fc);
-    else phase_initial(c);
+    else integrate_step(c);
     HIPCHK(hipEventRecord(E[4], c->stream));
     // next step's rebuild decision (Neighbor::decide): the atoms are final
     if (c->neigh_set) enqueue_decide(c, !last && c->lists_valid);
@@ -1333,8 +1353,8 @@ void run_steps_pipelined(phafd_hip_ctx *c, int nsteps, bool fused, bool zsplit, 
     const bool capture = c->fourier_capture && last;
     if (capture) capture_spectrum(c, 0, c->fields<R>().phihat.p);   // in_fourier: ft_phi before the update
     const bool next = next_ok && !last;
-    if (zsplit) phase_final_split<R>(c, !fc, next);
-    else phase_final_t<R>(c, !fc);
+    if (zsplit) phase_final_split<R>(c, false, next);
+    else phase_final_t<R>(c, false);
     HIPCHK(hipEventRecord(E[6], c->stream));
     if (zsplit) phase_postfinal_split<R>(c, next, phi0_slot(set));
     else phase_postfinal_t<R>(c);
@@ -1385,29 +1405,26 @@ void run_steps_t(phafd_hip_ctx *c, int nsteps) {
   c->grad_ready = false;
   FixDef *fc = fused_chain_fix(c);
   if (c->neigh_set) clear_decide_slot(c, c->timestep + 1);
-  // Pipelined steps: when every atom move of a step happens at
-  // initial_integrate (the fused chain fix, or no atom integrator), the next
-  // step's rebuild decision is known right after it.  The decision and the
-  // flags are then read back mid-step, and the host enqueues step k + 1
-  // while the device still runs step k's grid passes; the NaN check of step
-  // k's phi(0,0,0) happens once step k + 1 is enqueued (after PHAFD_E_NAN the
-  // fields hold one step more than the step reported).
-  bool atom_final = false;
-  for (auto &f : c->fixes)
-    if (f->kind != FixDef::CONJ && f->kind != FixDef::FH && f->kind != FixDef::GRADPHI && f.get() != fc)
-      atom_final = true;
-  if (!c->touch && !atom_final) {   // an active kernel probe collects its events after the run
+  // Pipelined steps: every atom move of a step is enqueued at
+  // initial_integrate (the hooks up to final_integrate work on the fields
+  // only), so the next step's rebuild decision is known right after it.  The
+  // decision and the flags are then read back mid-step, and the host enqueues
+  // step k + 1 while the device still runs step k's grid passes; the NaN check
+  // of step k's phi(0,0,0) happens once step k + 1 is enqueued (after
+  // PHAFD_E_NAN the fields hold one step more than the step reported).
+  if (!c->touch) {   // an active kernel probe collects its events after the run
     run_steps_pipelined<R>(c, nsteps, fused, zsplit, next_ok, pre, fc);
     return;
   }
-  bool started = false;   // this step's start_of_step went in before the last read-back
+  // run_until_touching: the chain ends are read back after every step, and
+  // the run may stop there
   for (int it = 0; it < nsteps; it++) {
-    if (!started) c->timestep++;
+    c->timestep++;
     const int64_t step = c->timestep;
     // muhat is observable only after the run: its last step stores it
     c->store_muhat = it == nsteps - 1;
     HIPCHK(hipEventRecord(c->ev[0], c->stream));
-    if (!started) phase_start(c);
+    phase_start(c);
     HIPCHK(hipEventRecord(c->ev[1], c->stream));
     phase_neigh(c);
     HIPCHK(hipEventRecord(c->ev[2], c->stream));
@@ -1422,11 +1439,10 @@ void run_steps_t(phafd_hip_ctx *c, int nsteps) {
     HIPCHK(hipEventRecord(c->ev[5], c->stream));
     const bool capture = c->fourier_capture && it == nsteps - 1;
     if (capture) capture_spectrum(c, 0, c->fields<R>().phihat.p);   // in_fourier: ft_phi before the update
-    const bool next = next_ok && it + 1 < nsteps;
-    if (zsplit) phase_final_split<R>(c, !fc, next);
+    if (zsplit) phase_final_split<R>(c, !fc);
     else phase_final_t<R>(c, !fc);
     HIPCHK(hipEventRecord(c->ev[6], c->stream));
-    if (zsplit) phase_postfinal_split<R>(c, next);
+    if (zsplit) phase_postfinal_split<R>(c);
     else phase_postfinal_t<R>(c);
     if (capture) {   // ft_chempot: the last step of a run stores the complete muhat
       capture_spectrum(c, 1, c->fields<R>().muhat.p);
@@ -1438,22 +1454,10 @@ void run_steps_t(phafd_hip_ctx *c, int nsteps) {
     if (c->neigh_set) enqueue_decide(c);
     enqueue_flags_readback(c);
     HIPCHK(hipMemcpyAsync(c->h_flags + 2, c->fields<R>().phi.p, sizeof(R), hipMemcpyDeviceToHost, c->stream));
-    if (c->touch) {   // the chain ends' positions after the step, read back with the flags
-      HIPCHK(hipMemcpyAsync(c->h_ends, c->x.p, sizeof(double4), hipMemcpyDeviceToHost, c->stream));
-      HIPCHK(hipMemcpyAsync(c->h_ends + 4, c->x.p + (c->nowned - 1), sizeof(double4), hipMemcpyDeviceToHost,
-                            c->stream));
-    }
+    // the chain ends' positions after the step, read back with the flags
+    HIPCHK(hipMemcpyAsync(c->h_ends, c->x.p, sizeof(double4), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(c->h_ends + 4, c->x.p + (c->nowned - 1), sizeof(double4), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipEventRecord(c->ev[8], c->stream));
-    // The next step's start_of_step (grad phi: the fields only, not the
-    // rebuild decision) goes in before the host waits for the read-back, so
-    // the device works through the host's turnaround.
-    started = it + 1 < nsteps && !c->touch;   // a touching run may stop after any step
-    if (started) {
-      c->timestep++;
-      HIPCHK(hipEventRecord(c->ev_pre[0], c->stream));
-      phase_start(c);
-      HIPCHK(hipEventRecord(c->ev_pre[1], c->stream));
-    }
     sync(c);
     probe_collect();
     for (int k = 0; k < 7; k++) {
@@ -1464,27 +1468,11 @@ void run_steps_t(phafd_hip_ctx *c, int nsteps) {
     float tot = 0;
     HIPCHK(hipEventElapsedTime(&tot, c->ev[0], c->ev[8]));
     c->tacc[7] += tot;
-    if (started) {
-      float ms = 0;
-      HIPCHK(hipEventElapsedTime(&ms, c->ev_pre[0], c->ev_pre[1]));
-      c->tacc[0] += ms;
-      c->tacc[7] += ms;
-    }
     R phi0;
     std::memcpy(&phi0, c->h_flags + 2, sizeof(R));
-    if (std::isnan(phi0) && started) c->timestep = step;   // the next step did not happen
-    if (std::isnan(phi0)) {
-      c->grad_ready = false;
-      throw std::runtime_error("NAN encountered in phi.");
-    }
-    try {
-      check_step_flags(c, step);
-    } catch (...) {
-      if (started) c->timestep = step;
-      c->grad_ready = false;
-      throw;
-    }
-    if (c->touch && touch_check(c, step, it + 1)) break;
+    if (std::isnan(phi0)) throw std::runtime_error("NAN encountered in phi.");
+    check_step_flags(c, step);
+    if (touch_check(c, step, it + 1)) break;
   }
 }
 
@@ -1688,7 +1676,6 @@ void init_ctx(phafd_hip_ctx *c, const phafd_hip_desc *desc, const MemberSlot *sl
     c->esum.alloc(8);
     HIPCHK(hipHostMalloc((void **)&c->h_flags, 128, hipHostMallocDefault));
     for (auto &e : c->ev) HIPCHK(hipEventCreate(&e));
-    for (auto &e : c->ev_pre) HIPCHK(hipEventCreate(&e));
     for (auto &set : c->evp)
       for (auto &e : set) HIPCHK(hipEventCreate(&e));
     for (int w = PHAFD_PHI; w <= PHAFD_GRADZ; w++)
@@ -1731,7 +1718,6 @@ int phafd_hip_destroy(phafd_hip_ctx *c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (auto &e : c->ev) if (e) (void)hipEventDestroy(e);
-  for (auto &e : c->ev_pre) if (e) (void)hipEventDestroy(e);
   for (auto &set : c->evp)
     for (auto &e : set) if (e) (void)hipEventDestroy(e);
   if (c->h_flags) (void)hipHostFree(c->h_flags);
