@@ -2840,15 +2840,22 @@ int phafd_hip_gradphi(int nx, int ny, int nz, const double *period, const double
     const size_t N = sc.plan.N(), M = sc.plan.M();
     DBuf<double> r, g[3];
     DBuf<double2> ph, gh[3];
-    r.alloc(N); ph.alloc(M);
-    for (int d = 0; d < 3; d++) { g[d].alloc(N); gh[d].alloc(M); }
+    r.alloc(N);
+    for (int d = 0; d < 3; d++) g[d].alloc(N);
     HIPCHK(hipMemcpy(r.p, phi, sizeof(double) * N, hipMemcpyHostToDevice));
-    fft_r2c(sc.plan, r.p, ph.p, sc.s);
     SpecConst k{2 * PI_REF / period[0], 2 * PI_REF / period[2], 2 * PI_REF / period[1]};
-    grad_multiply(sc.plan, ph.p, gh[0].p, gh[1].p, gh[2].p, k, sc.s);
-    double2 *ins[3] = {gh[0].p, gh[1].p, gh[2].p};
-    double *outs[3] = {g[0].p, g[1].p, g[2].p};
-    fft_c2r_batch(sc.plan, ins, outs, 3, (double)nx * ny * nz, sc.s);
+    if (fft_sep_grad_ok(sc.plan)) {
+      ph.alloc(2 * M);
+      fft_gradient(sc.plan, r.p, ph.p, g[0].p, g[1].p, g[2].p, k, sc.s);
+    } else {
+      ph.alloc(M);
+      for (int d = 0; d < 3; d++) gh[d].alloc(M);
+      fft_r2c(sc.plan, r.p, ph.p, sc.s);
+      grad_multiply(sc.plan, ph.p, gh[0].p, gh[1].p, gh[2].p, k, sc.s);
+      double2 *ins[3] = {gh[0].p, gh[1].p, gh[2].p};
+      double *outs[3] = {g[0].p, g[1].p, g[2].p};
+      fft_c2r_batch(sc.plan, ins, outs, 3, (double)nx * ny * nz, sc.s);
+    }
     HIPCHK(hipStreamSynchronize(sc.s));
     HIPCHK(hipMemcpy(gx, g[0].p, sizeof(double) * N, hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(gy, g[1].p, sizeof(double) * N, hipMemcpyDeviceToHost));

@@ -181,6 +181,10 @@ PHAFD_FFT_API(f64, double, double2)
 PHAFD_FFT_API(f32, float, float2)
 #undef PHAFD_FFT_API
 
+void fft_gradient(const FFTPlan &p, const double *phi, double2 *scratch, double *gx, double *gy, double *gz, SpecConst sc,
+                  hipStream_t s) {
+  f64::fft_gradient_p(p, phi, scratch, gx, gy, gz, sc, s);
+}
 bool fft_fused_z_ok(const FFTPlan &p) { return f64::fft_fused_z_ok_p(p); }
 bool fft_sep_grad_ok(const FFTPlan &p) { return f64::fft_sep_grad_ok_p(p); }
 

@@ -184,6 +184,9 @@ PHAFD_FFT_DECL(float, float2)
 #undef PHAFD_FFT_DECL
 bool fft_fused_z_ok(const FFTPlan &p);
 bool fft_sep_grad_ok(const FFTPlan &p);
+// the gradient of phi alone (grids with fft_sep_grad_ok), scratch: 2 M complex values
+void fft_gradient(const FFTPlan &p, const double *phi, double2 *scratch, double *gx, double *gy, double *gz, SpecConst sc,
+                  hipStream_t s);
 
 // ------------------------------------------------------------ field kernels
 struct SpecConst {

@@ -1,10 +1,11 @@
 // noalloc.hip -- grad(phi) without any device allocation.
 //
-// phafd_hip_gradphi_noalloc runs the kernels of phafd_hip_gradphi (the
-// r2c of phi, the i*q multiply, one c2r per component;
-// src/fixgrid_conjugate.cpp:62-116) on caller-owned device arrays.  Its
-// intermediates -- the half spectrum of phi and one gradient spectrum -- and
-// the FFT twiddle tables live in `scratch`, a static device array of
+// phafd_hip_gradphi_noalloc runs the kernels of phafd_hip_gradphi (the line
+// derivatives where the grid has them, else the r2c of phi, the i*q multiply
+// and one c2r per component; src/fixgrid_conjugate.cpp:62-116) on
+// caller-owned device arrays.  Its intermediates -- the alternating sums, or
+// the half spectrum of phi and one gradient spectrum -- and the FFT twiddle
+// tables live in `scratch`, a static device array of
 // PHAFD_NOALLOC_SCRATCH_BYTES that each GPU holds until the process ends:
 //
 //   [0, 64 KiB)        twiddles exp(-2 pi i m/L) at entry L-2 and
@@ -111,11 +112,15 @@ extern "C" int phafd_hip_gradphi_noalloc(int nx, int ny, int nz, const double *p
     double2 *ph = (double2 *)(base + TAB_BYTES);
     double2 *gh = ph + M;
     hipStream_t s = (hipStream_t)stream;
-    fft_r2c(plan, phi, ph, s);
     // SpecConst of phafd_hip_gradphi: x by 2 pi / period[0], y by
     // 2 pi / period[1], z by 2 pi / period[2] (PI of src/domain.cpp:206-208)
     const double PI_REF = 3.141592;
     const double dq[3] = {2 * PI_REF / period[0], 2 * PI_REF / period[1], 2 * PI_REF / period[2]};
+    if (fft_sep_grad_ok(plan)) {   // both spectra's room is the line kernels' scratch
+      fft_gradient(plan, phi, ph, gx, gy, gz, SpecConst{dq[0], dq[2], dq[1]}, s);
+      return PHAFD_OK;
+    }
+    fft_r2c(plan, phi, ph, s);
     double *out[3] = {gx, gy, gz};
     const unsigned blocks = (unsigned)std::min<size_t>((M + 255) / 256, 4096);
     for (int d = 0; d < 3; d++) {

@@ -41,3 +41,14 @@ def test_line_gradient(shape):
         s.run(3)   # the last step's gradient comes from the step before it
     for w in (P.GRADX, P.GRADY, P.GRADZ, P.PHI):
         assert rel_l2(g.get_field(w), o.get_field(w)) < 1e-12
+
+
+@pytest.mark.parametrize("shape", SHAPES + [(32, 64, 16), (64, 32, 16), (32, 64, 64), (128, 128, 128), (16, 8, 32)])
+def test_stateless_gradient(shape):
+    """phafd_hip_gradphi: the line kernels with the Nyquist terms from the
+    alternating sums (16 x 8 x 32: the transforms)."""
+    nx, ny, nz = shape
+    period = [0.9 * nx, 1.1 * ny, 1.3 * nz]
+    phi = P.ic_noisy_constant((nz, ny, nx), 0.45, 0.2, 78)
+    for a, b in zip(P.gradphi(phi, period), O.gradphi(phi, period)):
+        assert rel_l2(a, b) < 1e-12
