@@ -288,7 +288,8 @@ int phafd_hip_bins(phafd_hip_ctx *ctx, int *info, int *binhead, int *bins, int *
 int phafd_hip_energy(phafd_hip_ctx *ctx, double *out4);
 /* per-hook GPU time in ms accumulated over run() calls (hipEvent timers):
  * {gradphi, neighbor, pair, integrate, floryhuggins+r2c mu, update, c2r phi, total};
- * reset when reset != 0 */
+ * reset when reset != 0; integrate holds both halves of the atom integrators,
+ * which run() takes together at initial_integrate */
 int phafd_hip_timers(phafd_hip_ctx *ctx, double *ms8, int reset);
 /* run-time options (defaults in brackets):
  *  PHAFD_OPT_EAGER_GRIDLIST [0]: store the NPairGridBin list at every build
@@ -324,8 +325,10 @@ int phafd_hip_timers(phafd_hip_ctx *ctx, double *ms8, int reset);
  *  PHAFD_OPT_NEXT_GRADIENT [1]: inside phafd_hip_run, a step that another
  *    step follows also makes the next step's grad phi from its updated
  *    spectrum (the next r2c of phi is N times that spectrum in exact
- *    arithmetic, src/fixgrid_conjugate.cpp:62-154), so the next
- *    start_of_step transforms nothing; results agree with 0 to rounding.
+ *    arithmetic, src/fixgrid_conjugate.cpp:62-154; in FP64 above 2^18
+ *    points the y and z derivatives from phi's own lines and the
+ *    spectrum's Nyquist planes), so the next start_of_step has no
+ *    transform of phi; results agree with 0 to rounding.
  *    The last step of a run (and every step of run_until_touching) leaves
  *    the fields as the reference does. */
 enum { PHAFD_OPT_EAGER_GRIDLIST = 0, PHAFD_OPT_FUSE_FH = 1, PHAFD_OPT_FUSE_SPECTRAL = 2,
