@@ -502,7 +502,10 @@ int phafd_hip_spectral_update(int nx, int ny, int nz, const double *period, doub
  * serving loops, harnesses that forbid hipMalloc).  The gradient of
  * phafd_hip_gradphi, computed by the same kernels, on caller-owned DEVICE
  * arrays phi, gx, gy, gz (double[Nz][Ny][Nx]), enqueued on `stream` (a
- * hipStream_t; NULL: the null stream) and not waited for.  The
+ * hipStream_t; NULL: the null stream) and not waited for.  An output may be
+ * phi's own array, and outputs nobody needs may share one: phi is then read
+ * whole before the first output, and gx, gy, gz are written in this order (by
+ * the transforms instead of the line kernels; equal to rounding).  The
  * intermediates (two half spectra) and the FFT twiddles live in a static
  * device array of PHAFD_NOALLOC_SCRATCH_BYTES that each GPU holds until the
  * process ends; grids with (Nx/2+1)*Ny*Nz above

@@ -1,9 +1,9 @@
 // noalloc.hip -- grad(phi) without any device allocation.
 //
 // phafd_hip_gradphi_noalloc runs the kernels of phafd_hip_gradphi (the line
-// derivatives where the grid has them, else the r2c of phi, the i*q multiply
-// and one c2r per component; src/fixgrid_conjugate.cpp:62-116) on
-// caller-owned device arrays.  Its intermediates -- the alternating sums, or
+// derivatives where the grid has them, else, and where arrays of the caller
+// share memory, the r2c of phi, the i*q multiply and one c2r per component;
+// src/fixgrid_conjugate.cpp:62-116) on caller-owned device arrays.  Its intermediates -- the alternating sums, or
 // the half spectrum of phi and one gradient spectrum -- and the FFT twiddle
 // tables live in `scratch`, a static device array of
 // PHAFD_NOALLOC_SCRATCH_BYTES that each GPU holds until the process ends:
@@ -21,6 +21,8 @@
 // from the spectra it has written first, so nothing needs clearing; the
 // twiddles are never written again.  Calls share their GPU's array, so
 // calls that overlap on one GPU (other streams, other host threads) race.
+#include <algorithm>
+#include <cstdint>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -76,6 +78,18 @@ __global__ void k_grad_one(const double2 *__restrict__ ph, double2 *__restrict__
   }
 }
 
+// Whether any two of a call's four arrays of n doubles share memory.  The line
+// kernels read phi after they have written gx and write gy and gz in one
+// launch, so they need four separate arrays; the transforms have read the whole
+// of phi before they write gx, gy and gz one after the other.
+bool overlap(const double *phi, const double *gx, const double *gy, const double *gz, size_t n) {
+  uintptr_t a[4] = {(uintptr_t)phi, (uintptr_t)gx, (uintptr_t)gy, (uintptr_t)gz};
+  std::sort(a, a + 4);
+  for (int i = 0; i < 3; i++)
+    if (a[i + 1] - a[i] < n * sizeof(double)) return true;
+  return false;
+}
+
 }  // namespace
 
 namespace phafd {
@@ -116,7 +130,7 @@ extern "C" int phafd_hip_gradphi_noalloc(int nx, int ny, int nz, const double *p
     // 2 pi / period[1], z by 2 pi / period[2] (PI of src/domain.cpp:206-208)
     const double PI_REF = 3.141592;
     const double dq[3] = {2 * PI_REF / period[0], 2 * PI_REF / period[1], 2 * PI_REF / period[2]};
-    if (fft_sep_grad_ok(plan)) {   // both spectra's room is the line kernels' scratch
+    if (fft_sep_grad_ok(plan) && !overlap(phi, gx, gy, gz, N)) {   // both spectra's room is the line kernels' scratch
       fft_gradient(plan, phi, ph, gx, gy, gz, SpecConst{dq[0], dq[2], dq[1]}, s);
       return PHAFD_OK;
     }
