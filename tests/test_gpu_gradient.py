@@ -52,3 +52,18 @@ def test_stateless_gradient(shape):
     phi = P.ic_noisy_constant((nz, ny, nx), 0.45, 0.2, 78)
     for a, b in zip(P.gradphi(phi, period), O.gradphi(phi, period)):
         assert rel_l2(a, b) < 1e-12
+
+
+@pytest.mark.parametrize("shape", [(32, 16, 16), (64, 32, 64), (128, 128, 128), (16, 8, 32)])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_stateless_gradient_of_a_field_with_a_hole(shape, value):
+    """One NaN or infinity in phi, at the first, the last and an inner point:
+    nothing of the gradient is finite, as after a transform in three dimensions
+    (16 x 8 x 32)."""
+    nx, ny, nz = shape
+    phi = P.ic_noisy_constant((nz, ny, nx), 0.45, 0.2, 79)
+    for at in ((0, 0, 0), (nz - 1, ny - 1, nx - 1), (nz // 2 + 1, 5, 3)):
+        bad = phi.copy()
+        bad[at] = value
+        for g in P.gradphi(bad, [1.0 * nx, 1.0 * ny, 1.0 * nz]):
+            assert not np.isfinite(g).any()
