@@ -255,7 +255,10 @@ int phafd_hip_fix_semiflexible(phafd_hip_ctx *ctx, int tether, int nchunk, const
  *      (src/neighbor.cpp:39-68, src/comm_brick.cpp:96-187) */
 int phafd_hip_neighbor(phafd_hip_ctx *ctx, double skin);
 
-/* ---- run: Integrate::setup / Integrate::run (src/integrate.cpp:33-219) */
+/* ---- run: Integrate::setup / Integrate::run (src/integrate.cpp:33-219).
+ * After PHAFD_E_NAN the positions (wrapped into the box where the next step
+ * rebuilds its lists) and forces are those of the step reported; the fields
+ * may hold one step more, which was enqueued before the check. */
 int phafd_hip_setup(phafd_hip_ctx *ctx, double dt);
 int phafd_hip_run(phafd_hip_ctx *ctx, int nsteps);
 /* one hook phase of a timestep (PHAFD_PH_*); PHAFD_PH_START advances the step */

@@ -24,8 +24,9 @@ int nblk(size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < (size_t)(n); i += (size_t)gridDim.x * blockDim.x)
 
 // a kernel of a speculative window's step that follows the step whose
-// rebuild decision fired (StepGate)
+// rebuild decision fired, or of a step that follows one that left NaN (StepGate)
 __device__ __forceinline__ bool gate_off(const StepGate &g) {
+  if (g.phi && (g.f32 ? isnan(*(const float *)g.phi) : isnan(*(const double *)g.phi))) return true;
   if (!g.stop) return false;
   const int t = *g.stop;
   return t > 0 && g.step > t;
@@ -1214,7 +1215,8 @@ __global__ __launch_bounds__(256) void k_fill_multi(const FoldDev *__restrict__ 
 // ---------------------------------------------------------- integrators
 // FixAtomDrag half step, src/fixatom_drag.cpp:43-66
 __global__ void k_drag(int n, const int *members, double4 *x, const double4 *F, double drag,
-                       double dt, int halves) {
+                       double dt, int halves, StepGate gate) {
+  if (gate_off(gate)) return;
   GRID_STRIDE(q, n) {
     const int j = members[q];
     double4 p = x[j];
@@ -1539,7 +1541,8 @@ __device__ __forceinline__ double4 br_map(double x, double y, double z, int img,
 // FixAtomSemiFlexible::initial_integrate -> first_step
 __global__ __launch_bounds__(64) void k_br_first(const int *chs, const int *che, const int *seeds, const double4 *F,
                                                  double4 *ux, double4 *x, const int *image, double4 *R0,
-                                                 double4 *FB, double *Tg, BRParamsDev p, Box bx, int L) {
+                                                 double4 *FB, double *Tg, BRParamsDev p, Box bx, int L, StepGate gate) {
+  if (gate_off(gate)) return;
   extern __shared__ double sh[];
   BRLds S;
   S.carve(sh, L);
@@ -1625,7 +1628,8 @@ __global__ __launch_bounds__(64) void k_br_first(const int *chs, const int *che,
 __global__ __launch_bounds__(64) void k_br_second(const int *chs, const int *che, const double4 *F, double4 *ux,
                                                   double4 *x, const int *image, const double4 *R0,
                                                   const double4 *FB, double *Tg, int *fail, BRParamsDev p, Box bx,
-                                                  int L) {
+                                                  int L, StepGate gate) {
+  if (gate_off(gate)) return;
   extern __shared__ double sh[];
   BRLds S;
   S.carve(sh, L);
@@ -1717,7 +1721,10 @@ __global__ __launch_bounds__(64) void k_br_second(const int *chs, const int *che
 }
 
 __global__ void k_fill_i32(int n, int *p, int v) { GRID_STRIDE(i, n) p[i] = v; }
-__global__ void k_fill_d4(int n, double4 *p) { GRID_STRIDE(i, n) p[i] = make_double4(0, 0, 0, 0); }
+__global__ void k_fill_d4(int n, double4 *p, StepGate gate) {
+  if (gate_off(gate)) return;
+  GRID_STRIDE(i, n) p[i] = make_double4(0, 0, 0, 0);
+}
 
 }  // namespace
 
@@ -2061,9 +2068,9 @@ void launch_harmonic_force(int ng, const HarmParams &h, const double4 *gx, const
   HIPCHK(hipGetLastError());
 }
 void launch_drag(int n, const int *members, double4 *x, const double4 *F, double drag, double dt,
-                 hipStream_t s, int halves) {
+                 hipStream_t s, int halves, StepGate gate) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_drag, dim3(nblk(n)), dim3(TPB), 0, s, n, members, x, F, drag, dt, halves);
+  hipLaunchKernelGGL(k_drag, dim3(nblk(n)), dim3(TPB), 0, s, n, members, x, F, drag, dt, halves, gate);
   HIPCHK(hipGetLastError());
 }
 void launch_chain_step(int nchains, int maxlen, const int *chs, const int *che, const double4 *F, double4 *ux,
@@ -2088,24 +2095,24 @@ void br_lds_allow(const void *k, size_t bytes) {
 }
 void launch_br_first(int nchains, int maxlen, const int *chs, const int *che, const int *seeds, const double4 *F,
                      double4 *ux, double4 *x, const int *image, double4 *R0, double4 *FB, double *T,
-                     const BRParamsDev &p, const Box &b, hipStream_t s) {
+                     const BRParamsDev &p, const Box &b, hipStream_t s, StepGate gate) {
   if (nchains <= 0 || maxlen <= 0) return;
   if (maxlen > BR_MAXLEN) throw std::invalid_argument("bead-rod chains longer than 700 beads are not supported");
   const size_t lds = br_lds_bytes(maxlen);
   br_lds_allow((const void *)k_br_first, lds);
   hipLaunchKernelGGL(k_br_first, dim3(nchains), dim3(64), lds, s, chs, che, seeds, F, ux, x, image, R0, FB, T, p, b,
-                     maxlen);
+                     maxlen, gate);
   HIPCHK(hipGetLastError());
 }
 void launch_br_second(int nchains, int maxlen, const int *chs, const int *che, const double4 *F, double4 *ux,
                       double4 *x, const int *image, const double4 *R0, const double4 *FB, double *T, int *fail,
-                      const BRParamsDev &p, const Box &b, hipStream_t s) {
+                      const BRParamsDev &p, const Box &b, hipStream_t s, StepGate gate) {
   if (nchains <= 0 || maxlen <= 0) return;
   if (maxlen > BR_MAXLEN) throw std::invalid_argument("bead-rod chains longer than 700 beads are not supported");
   const size_t lds = br_lds_bytes(maxlen);
   br_lds_allow((const void *)k_br_second, lds);
   hipLaunchKernelGGL(k_br_second, dim3(nchains), dim3(64), lds, s, chs, che, F, ux, x, image, R0, FB, T, fail, p,
-                     b, maxlen);
+                     b, maxlen, gate);
   HIPCHK(hipGetLastError());
 }
 // the batched pair phase: grids of at most 8 blocks per CU take the items
@@ -2172,9 +2179,9 @@ void launch_fill_i32(int n, int *p, int v, hipStream_t s) {
   hipLaunchKernelGGL(k_fill_i32, dim3(nblk(n)), dim3(TPB), 0, s, n, p, v);
   HIPCHK(hipGetLastError());
 }
-void launch_fill_d4(int n, double4 *p, hipStream_t s) {
+void launch_fill_d4(int n, double4 *p, hipStream_t s, StepGate gate) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_fill_d4, dim3(nblk(n)), dim3(TPB), 0, s, n, p);
+  hipLaunchKernelGGL(k_fill_d4, dim3(nblk(n)), dim3(TPB), 0, s, n, p, gate);
   HIPCHK(hipGetLastError());
 }
 

@@ -40,9 +40,14 @@ struct GAParams {
 // Speculative windows of atom steps: stop (device) holds the 1-based step
 // of the window whose rebuild decision fired (0: none); the kernels of a
 // later step of the window return at once.  step 0 / stop null: not gated.
+// Steps enqueued before the one ahead of them is checked: phi (device) holds
+// the field that one left, FP32 where f32 is set; if its first value is NaN
+// the run ended there, and the kernels of the later step return at once.
 struct StepGate {
   int *stop = nullptr;
   int step = 0;
+  const void *phi = nullptr;
+  bool f32 = false;
 };
 
 struct LJParams {
@@ -166,7 +171,7 @@ void launch_harmonic_force(int ng, const HarmParams &h, const double4 *gx, const
                            const int *hneigh, const int *toff, const int *tpair, const int *ti, int nowned,
                            double4 *gF, hipStream_t s, bool zero_init = false, StepGate gate = StepGate());
 void launch_drag(int n, const int *members, double4 *x, const double4 *F, double drag, double dt,
-                 hipStream_t s, int halves = 1);
+                 hipStream_t s, int halves = 1, StepGate gate = StepGate());
 // halves (1 or 2) half steps of the chains (contiguous atom ranges
 // [chs[c], che[c]), at most maxlen beads, halves * maxlen * 32 bytes of LDS
 // per block); 2: both halves of a timestep, with the same F
@@ -246,13 +251,13 @@ struct BRParamsDev {
 // (first-order tensions) kept per atom for second_step
 void launch_br_first(int nchains, int maxlen, const int *chs, const int *che, const int *seeds, const double4 *F,
                      double4 *ux, double4 *x, const int *image, double4 *R0, double4 *FB, double *T,
-                     const BRParamsDev &p, const Box &b, hipStream_t s);
+                     const BRParamsDev &p, const Box &b, hipStream_t s, StepGate gate = StepGate());
 // second_step: ux (R* -> R1), x = map(ux); fail |= 1 past itermax iterations
 void launch_br_second(int nchains, int maxlen, const int *chs, const int *che, const double4 *F, double4 *ux,
                       double4 *x, const int *image, const double4 *R0, const double4 *FB, double *T, int *fail,
-                      const BRParamsDev &p, const Box &b, hipStream_t s);
+                      const BRParamsDev &p, const Box &b, hipStream_t s, StepGate gate = StepGate());
 void launch_fill_i32(int n, int *p, int v, hipStream_t s);
-void launch_fill_d4(int n, double4 *p, hipStream_t s);
+void launch_fill_d4(int n, double4 *p, hipStream_t s, StepGate gate = StepGate());
 void launch_add4(int n, const double4 *a, double4 *b, hipStream_t s);   // b.xyz += a.xyz
 
 }  // namespace phafd

@@ -437,23 +437,23 @@ void forward_comm(phafd_hip_ctx *c, StepGate gate = StepGate()) {
 // and the last fold are one pass; the sums are those of copy + reverse_comm
 void reverse_comm_from(phafd_hip_ctx *c, const double4 *init, StepGate gate = StepGate());
 
-void reverse_comm(phafd_hip_ctx *c) {
+void reverse_comm(phafd_hip_ctx *c, StepGate gate = StepGate()) {
   if (c->fold_tree) {
-    launch_fold_tree(c->nowned, c->fold_idx.p, c->fold_slot.p, c->gF.p, c->F.p, c->F.p, c->stream);
+    launch_fold_tree(c->nowned, c->fold_idx.p, c->fold_slot.p, c->gF.p, c->F.p, c->F.p, c->stream, gate);
     return;
   }
   for (int iswap = (int)c->swaps.size() - 1; iswap >= 1; iswap--) {
     SwapDev &w = c->swaps[iswap];
     if (w.disjoint_pair) {   // the dimension's two swaps in one launch (same sums)
       SwapDev &v = c->swaps[iswap - 1];
-      launch_reverse2(w.count, w.send.p, w.first, v.count, v.send.p, v.first, c->gF.p, c->stream);
+      launch_reverse2(w.count, w.send.p, w.first, v.count, v.send.p, v.first, c->gF.p, c->stream, gate);
       iswap--;
       continue;
     }
-    launch_reverse(w.count, w.send.p, w.first, c->gF.p, c->gF.p, c->stream);
+    launch_reverse(w.count, w.send.p, w.first, c->gF.p, c->gF.p, c->stream, gate);
   }
   SwapDev &z = c->swaps[0];
-  launch_reverse(z.count, z.send.p, z.first, c->F.p, c->gF.p, c->stream);
+  launch_reverse(z.count, z.send.p, z.first, c->F.p, c->gF.p, c->stream, gate);
 }
 
 bool reverse_from_one_pass(const phafd_hip_ctx *c) { return c->swaps[0].count == c->nowned; }
@@ -1005,7 +1005,9 @@ void grid_atom_pass(phafd_hip_ctx *c, PairDef &p, double *energy, bool first, bo
 }
 
 // Integrate::run pair block, src/integrate.cpp:130-146 (one pass, finding F4)
-void phase_pair(phafd_hip_ctx *c, double *energy_ga = nullptr, double *energy_lj = nullptr) {
+// gate: leaves F alone
+void phase_pair(phafd_hip_ctx *c, double *energy_ga = nullptr, double *energy_lj = nullptr,
+                StepGate gate = StepGate()) {
   // mu = 0 before the pair computes: done by the first grid-atom pass, which
   // writes every grid point, when there is one
   bool mu_pending = true;
@@ -1021,7 +1023,7 @@ void phase_pair(phafd_hip_ctx *c, double *energy_ga = nullptr, double *energy_lj
   const bool lists = c->neigh_set && c->lists_valid;
   bool gf_pending = lists && !c->pairs.empty();
   if (!gf_pending) launch_fill_d4(c->ngathered, c->gF.p, c->stream);
-  if (!lists || !c->fold_tree) launch_fill_d4(c->nowned, c->F.p, c->stream);
+  if (!lists || !c->fold_tree) launch_fill_d4(c->nowned, c->F.p, c->stream, gate);
   if (!lists) return;
   for (auto &pp : c->pairs) {
     PairDef &p = *pp;
@@ -1041,36 +1043,36 @@ void phase_pair(phafd_hip_ctx *c, double *energy_ga = nullptr, double *energy_lj
     }
     gf_pending = false;
   }
-  if (c->fold_tree) reverse_comm_from(c, nullptr);
-  else reverse_comm(c);
+  if (c->fold_tree) reverse_comm_from(c, nullptr, gate);
+  else reverse_comm(c, gate);
 }
 
 // second: the final_integrate half (FixAtomDrag and the harmonic chains do
 // the same in both halves; the bead-rod fix runs first_step, then second_step)
-void integrate_half(phafd_hip_ctx *c, FixDef &f, bool second = false) {
+void integrate_half(phafd_hip_ctx *c, FixDef &f, bool second = false, StepGate gate = StepGate()) {
   if (f.kind == FixDef::SEMIFLEX) {
     BRParamsDev p{f.bondlength, f.zpar, f.zperp, f.bending, f.brtemp, c->dt, f.tether, 50, f.brstep};
     if (!second) {
       p.step = ++f.brstep;
       launch_br_first(f.nchain, f.maxlen, f.chs.p, f.che.p, f.d_seed.p, c->F.p, c->ux.p, c->x.p, c->image.p,
-                      f.br_R0.p, f.br_FB.p, f.br_T.p, p, c->box(), c->stream);
+                      f.br_R0.p, f.br_FB.p, f.br_T.p, p, c->box(), c->stream, gate);
     } else {
       launch_br_second(f.nchain, f.maxlen, f.chs.p, f.che.p, c->F.p, c->ux.p, c->x.p, c->image.p, f.br_R0.p,
-                       f.br_FB.p, f.br_T.p, c->flags.p + 3, p, c->box(), c->stream);
+                       f.br_FB.p, f.br_T.p, c->flags.p + 3, p, c->box(), c->stream, gate);
     }
     return;
   }
   if (f.kind == FixDef::DRAG) {
-    launch_drag(f.nmem, f.members.p, c->x.p, c->F.p, f.drag, c->dt, c->stream);
+    launch_drag(f.nmem, f.members.p, c->x.p, c->F.p, f.drag, c->dt, c->stream, 1, gate);
   } else if (f.kind == FixDef::CHAIN) {
     ChainParams cp{f.r0, f.kbond, f.kbend, f.drag};
     launch_chain_step(f.nchain, f.maxlen, f.chs.p, f.che.p, c->F.p, c->ux.p, c->x.p, c->image.p, cp, c->dt,
-                      c->box(), c->stream);
+                      c->box(), c->stream, 1, gate);
   }
 }
 
-void phase_initial(phafd_hip_ctx *c) {
-  for (auto &f : c->fixes) integrate_half(c, *f);
+void phase_initial(phafd_hip_ctx *c, StepGate gate = StepGate()) {
+  for (auto &f : c->fixes) integrate_half(c, *f, false, gate);
 }
 
 // Both half steps of every atom integrator, at initial_integrate.  F is made
@@ -1078,7 +1080,7 @@ void phase_initial(phafd_hip_ctx *c) {
 // final_integrate work on the fields only, so the positions are those of the
 // halves in their places; the first halves of all fixes come before the
 // second ones, as there.
-void integrate_step(phafd_hip_ctx *c) {
+void integrate_step(phafd_hip_ctx *c, StepGate gate) {
   FixDef *one = nullptr;
   int n = 0;
   for (auto &f : c->fixes)
@@ -1087,11 +1089,11 @@ void integrate_step(phafd_hip_ctx *c) {
       n++;
     }
   if (n == 1 && one->kind == FixDef::DRAG) {   // nothing between its halves
-    launch_drag(one->nmem, one->members.p, c->x.p, c->F.p, one->drag, c->dt, c->stream, 2);
+    launch_drag(one->nmem, one->members.p, c->x.p, c->F.p, one->drag, c->dt, c->stream, 2, gate);
     return;
   }
-  phase_initial(c);
-  for (auto &f : c->fixes) integrate_half(c, *f, true);
+  phase_initial(c, gate);
+  for (auto &f : c->fixes) integrate_half(c, *f, true, gate);
 }
 
 // The chain fix when it is the only atom integrator (and its chains fit two
@@ -1283,6 +1285,21 @@ void capture_spectrum(phafd_hip_ctx *c, int k, const float2 *src) {
   HIPCHK(hipGetLastError());
 }
 
+// what a step takes from its fixes' random streams: the queued noise fields'
+// head and every bead-rod fix's counter; put_back: as before that step
+std::vector<unsigned long long> draws(const phafd_hip_ctx *c) {
+  std::vector<unsigned long long> v{c->noise_head};
+  for (auto &f : c->fixes)
+    if (f->kind == FixDef::SEMIFLEX) v.push_back(f->brstep);
+  return v;
+}
+void put_back(phafd_hip_ctx *c, const std::vector<unsigned long long> &v) {
+  size_t k = 0;
+  c->noise_head = v[k++];
+  for (auto &f : c->fixes)
+    if (f->kind == FixDef::SEMIFLEX) f->brstep = v[k++];
+}
+
 // see run_steps_t: the steps with the flags read back mid-step, step k + 1
 // enqueued before step k ends
 template <class R>
@@ -1297,6 +1314,7 @@ void run_steps_pipelined(phafd_hip_ctx *c, int nsteps, bool fused, bool zsplit, 
     bool &f;
     ~Ahead() { f = false; }
   } ahead{c->gx_ahead};
+  std::vector<unsigned long long> drawn;   // draws() before the latest step
   // the timers and the NaN check of a completed step
   auto finish = [&](int set, int64_t step) {
     hipEvent_t *E = c->evp[set];
@@ -1312,6 +1330,7 @@ void run_steps_pipelined(phafd_hip_ctx *c, int nsteps, bool fused, bool zsplit, 
     std::memcpy(&phi0, phi0_slot(set), sizeof(R));
     if (std::isnan(phi0)) {
       sync(c);   // a later step in flight ends first
+      if (c->timestep != step) put_back(c, drawn);
       c->timestep = step;
       c->grad_ready = false;
       c->pending_decision = -1;
@@ -1327,15 +1346,30 @@ void run_steps_pipelined(phafd_hip_ctx *c, int nsteps, bool fused, bool zsplit, 
     const int64_t step = c->timestep;
     const bool last = it == nsteps - 1;
     c->store_muhat = last;
+    // the atoms move only if the step before, unchecked so far, left no NaN
+    StepGate gate;
+    if (prev_step >= 0) {
+      gate.phi = c->fields<R>().phi.p;
+      gate.f32 = sizeof(R) == sizeof(float);
+    }
+    drawn = draws(c);
     HIPCHK(hipEventRecord(E[0], c->stream));
     phase_start(c);
     HIPCHK(hipEventRecord(E[1], c->stream));
-    phase_neigh(c);
+    try {
+      phase_neigh(c);
+    } catch (...) {
+      if (prev_step >= 0) {   // a NaN of the step before comes first
+        sync(c);
+        finish(set ^ 1, prev_step);
+      }
+      throw;
+    }
     HIPCHK(hipEventRecord(E[2], c->stream));
-    phase_pair(c);
+    phase_pair(c, nullptr, nullptr, gate);
     HIPCHK(hipEventRecord(E[3], c->stream));
-    if (fc) integrate_both_halves(c, *fc);
-    else integrate_step(c);
+    if (fc) integrate_both_halves(c, *fc, gate);
+    else integrate_step(c, gate);
     HIPCHK(hipEventRecord(E[4], c->stream));
     // next step's rebuild decision (Neighbor::decide): the atoms are final
     if (c->neigh_set) enqueue_decide(c, !last && c->lists_valid);
@@ -1410,8 +1444,10 @@ void run_steps_t(phafd_hip_ctx *c, int nsteps) {
   // only), so the next step's rebuild decision is known right after it.  The
   // decision and the flags are then read back mid-step, and the host enqueues
   // step k + 1 while the device still runs step k's grid passes; the NaN check
-  // of step k's phi(0,0,0) happens once step k + 1 is enqueued (after
-  // PHAFD_E_NAN the fields hold one step more than the step reported).
+  // of step k's phi(0,0,0) happens once step k + 1 is enqueued, so after
+  // PHAFD_E_NAN the fields may hold one step more than the step reported; the
+  // atoms and the forces on them do not, those of step k + 1 are gated on
+  // step k's phi (StepGate).
   if (!c->touch) {   // an active kernel probe collects its events after the run
     run_steps_pipelined<R>(c, nsteps, fused, zsplit, next_ok, pre, fc);
     return;
