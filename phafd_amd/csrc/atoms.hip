@@ -6,6 +6,7 @@
 // reference's exact expressions (built with -ffp-contract=off), so lists and
 // bins are bit-identical to the reference's on the same positions.
 #include "atoms.hpp"
+#include "segments.hpp"
 #include "spectral_ops.hpp"
 
 namespace phafd {
@@ -809,7 +810,7 @@ __global__ __launch_bounds__(256) void k_ga_pm_rank(int nent, const int *__restr
     const int p = ps[e].x, q = amq[e];
     const int s = poff[p], t = poff[p + 1];
     int n = 0, i = s;
-    for (; i + 4 <= t; i += 4) {
+    for (; t - i >= 4; i += 4) {
       const int k0 = key[i], k1 = key[i + 1], k2 = key[i + 2], k3 = key[i + 3];
       n += (k0 < q) + (k1 < q) + (k2 < q) + (k3 < q);
     }
@@ -864,13 +865,13 @@ __device__ __forceinline__ void ga_force_atom(size_t q, bool on, const GridViewT
                                               double &esum, bool want_energy, int lx, int lxy) {
   const int mx = gv.nx - 1, my = gv.ny - 1;
   const int lane = threadIdx.x & 63, sub = lane & (G - 1), first = lane & ~(G - 1);
-  int c = 0, e = 0, a = 0;
+  LaneWalk w(0, 0, 0);
+  int a = 0;
   if (on) {
-    c = aoff[q] + sub;
-    e = aoff[q + 1];
+    w = LaneWalk(aoff[q], aoff[q + 1], sub);
     a = order[q];
   }
-  int2 nx = c < e ? ps[c] : make_int2(0, 0);
+  int2 nx = w.on() ? ps[w.c] : make_int2(0, 0);
   double4 x = make_double4(0.0, 0.0, 0.0, 0.0);
   if (on) x = gx[a];
   const int t = (int)x.w;
@@ -880,11 +881,11 @@ __device__ __forceinline__ void ga_force_atom(size_t q, bool on, const GridViewT
   ForceSum<R> acc;
   acc.F = 0.0;
   if (!ZI && on && sub < 3) acc.F = Fa[sub];
-  while (__any(c < e)) {
-    const bool act = c < e;
+  while (__any(w.on())) {
+    const bool act = w.on();
     const int p = nx.x, so = nx.y;
-    c += G;
-    nx = c < e ? ps[c] : make_int2(0, 0);   // the next pairs load while these terms are formed
+    w.next(G);
+    nx = w.on() ? ps[w.c] : make_int2(0, 0);   // the next pairs load while these terms are formed
     const int k = p & mx, j = (p >> lx) & my, i = p >> lxy;
     const double delz = (i * gv.dz + gv.lo[2]) - x.z;
     const double dely = (j * gv.dy + gv.lo[1]) - x.y;
@@ -1020,11 +1021,11 @@ __device__ __forceinline__ void ga_list_mu_block(size_t blk, size_t N, R *__rest
   }
   const size_t p1 = p0 + 256 * U < N ? p0 + 256 * U : N;
   const int b = poff[p0], t = poff[p1];
-  for (int c0 = b; c0 < t; c0 += GM_CH) {
-    const int c1 = t - c0 < GM_CH ? t : c0 + GM_CH;
+  for (int c0 = b, c1; c0 < t; c0 = c1) {
+    c1 = chunk_end(c0, t, GM_CH);
 #pragma unroll
     for (int i = 0; i < GM_CH; i += 256)
-      if (c0 + i + tid < c1) st[i + tid] = mterm[c0 + i + tid];
+      if (i + tid < c1 - c0) st[i + tid] = mterm[c0 + i + tid];
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < U; u++) {
