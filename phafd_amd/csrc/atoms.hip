@@ -329,10 +329,10 @@ __device__ __forceinline__ double4 fold_atom(size_t i, const int *__restrict__ i
   }
   return b;
 }
-// F = init (null: zero) + the folded gF
+// F = init (null: zero; F itself: added to) + the folded gF
 __global__ __launch_bounds__(256) void k_fold_tree(int n, const int *__restrict__ idx, const int *__restrict__ slot,
-                                                   const double4 *__restrict__ gF, const double4 *__restrict__ init,
-                                                   double4 *__restrict__ F, StepGate gate) {
+                                                   const double4 *__restrict__ gF, const double4 *init, double4 *F,
+                                                   StepGate gate) {
   if (gate_off(gate)) return;
   GRID_STRIDE(i, n) {
     double4 t = init ? init[i] : make_double4(0.0, 0.0, 0.0, 0.0);

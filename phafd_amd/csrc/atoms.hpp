@@ -92,7 +92,7 @@ void launch_reverse2(int ca, const int *sa, int fa, int cb, const int *sb, int f
                      StepGate gate = StepGate());
 // reverse comm as one fold per owned atom, where each owned atom is its own
 // LOCAL copy entry and the swaps of a dimension are disjoint: the image lists
-// of a build (idx: n, slot: 8 per ghost entry), and F = init (null: zero) +
+// of a build (idx: n, slot: 8 per ghost entry), and F = init (null: zero; may be F) +
 // the atom's gF with its images folded in, the sums of the swap by swap folds
 void launch_fold_lists(int n, int nghost, const GatheredView &g, int *idx, int *slot, hipStream_t s);
 void launch_fold_tree(int n, const int *idx, const int *slot, const double4 *gF, const double4 *init, double4 *F,
@@ -232,9 +232,10 @@ void launch_lj_multi(int nm, const LJMemberDev *d, const int *boff, int nitems, 
                      hipStream_t s);
 void launch_fold_multi(int nm, const FoldDev *d, const int *boff, int nitems, bool zero, const MultiShape &sh,
                        hipStream_t s);
-// target[0 .. ca) = 0 of every member
+// the one-launch fold of every member (sa: idx, sb: slot), F from zero
 void launch_fold_tree_multi(int nm, const FoldDev *d, const int *boff, int nitems, const MultiShape &sh,
                             hipStream_t s);
+// target[0 .. ca) = 0 of every member
 void launch_fill_multi(int nm, const FoldDev *d, const int *boff, int nitems, const MultiShape &sh, hipStream_t s);
 // both half steps of the harmonic chains of every member (coff: chain offsets)
 void launch_chain_multi(int nm, const ChainMemberDev *d, const int *coff, int nchains, int maxlen, double dt,

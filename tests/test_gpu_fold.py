@@ -42,3 +42,32 @@ def test_forces_of_folded_images(kind, n, box, zghost):
         for ph in (P.PH_START, P.PH_NEIGH, P.PH_PAIR):
             s.phase(ph)
     assert rel_l2(g.get_forces(), o.get_forces()) < 1e-10
+
+
+@pytest.mark.parametrize("zghost", [0, 1])
+@pytest.mark.parametrize("kind,n,box", [("corner", 16, 16.0), ("edges", 32, 32.0), ("all", 32, 32.0), ("all", 16, 8.0),
+                                        ("corner", 16, 4.0)])   # the last: images along both ways, no one-launch fold
+def test_folded_sums_are_the_swaps_bitwise(kind, n, box, zghost):
+    """lj/cut forces (products and quotients only, no function whose rounding
+    is the library's own) folded image by image in the oracle, swap after swap:
+    the same sums in the same order give the same bits."""
+    rng = np.random.default_rng(n + 1)
+    xyz = _beads(kind, box, rng)
+    out = []
+    for M, gpu in ((P, True), (O, False)):
+        s = M.System(n, n, n, [0, 0, 0], [box] * 3, zghost=zghost)
+        s.set_field(P.PHI, P.ic_noisy_constant((n, n, n), 0.4, 0.1, 5))
+        s.set_atoms(xyz, np.zeros(len(xyz), np.int32), tags=np.arange(len(xyz), dtype=np.int32),
+                    mols=np.zeros(len(xyz), np.int32))
+        if gpu:
+            s.pair_ljcut(2.0, 1.0, 1.0)
+        else:
+            s.add_pair(O.PAIR_LJCUT, 2.0, 1.0, 1.0)
+        s.fix_conjugate(5678, 1.0, 1.0, 1.0, 1.0, 0)
+        s.neighbor(0.4)
+        s.setup(1e-3)
+        for ph in (P.PH_START, P.PH_NEIGH, P.PH_PAIR):
+            s.phase(ph)
+        out.append(s.get_forces())
+    assert np.abs(out[0]).max() > 0
+    assert np.array_equal(*out)
