@@ -187,7 +187,7 @@ struct GAMemberDev {
   GridViewT<double> gv;
   GAParams ga;
   const double4 *gx;
-  const int *order, *aoff;
+  const int *order, *perm, *aoff;   // perm: the atoms tile by tile, or null
   const int2 *ps;
   double *mterm;
   double4 *gF;

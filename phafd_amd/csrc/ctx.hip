@@ -3208,7 +3208,8 @@ void batch_pair_fused(phafd_hip_batch *b, bool with_chains) {
     GAMemberDev &g = ga[i];
     g.gv = c->gridview<double>();
     g.ga = ga_params(*pga);
-    g.gx = c->gx.p; g.order = c->binatoms.p; g.aoff = c->ga_aoff.p; g.ps = c->ga_ps.p;
+    g.gx = c->gx.p; g.order = c->binatoms.p; g.perm = c->ga_tiled ? c->ga_perm.p : nullptr;
+    g.aoff = c->ga_aoff.p; g.ps = c->ga_ps.p;
     g.mterm = c->ga_mterm.p; g.gF = c->gF.p; g.ng = c->ngathered;
     g.mu = c->fd.mu.p; g.poff = c->ga_poff.p;
     boff_ga[i + 1] = boff_ga[i] + (c->ngathered + T - 1) / T;

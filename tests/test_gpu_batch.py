@@ -90,6 +90,23 @@ def test_one_launch_per_pass_matches_per_member_launches_bitwise(n):
     m.close()
 
 
+def test_wide_couplings_match_solo_runs_bitwise():
+    """Members whose walk takes the atoms by tiles of bins, one beside them
+    whose coupling is narrow, through the launch they share."""
+    ws = [workload(n=64, nchains=20, nbeads=20, seed=41 + i, ljish=i == 1, nucwidth=(2.5, 1.0, 2.25)[i])
+          for i in range(3)]
+    b = _batch(ws)
+    b.set_fused(1)
+    b.run(6)
+    for i, w in enumerate(ws):
+        s = make_gpu(w)
+        s.set_option(P.OPT_NEXT_GRADIENT, 0)
+        s.run(6)
+        _assert_same(_state(b.member(i)), _state(s), f"member {i}")
+        s.close()
+    b.close()
+
+
 def test_graphs_match_eager_launches_bitwise():
     ws = _members(64, 4)
     g = _batch(ws, graphs=True)
