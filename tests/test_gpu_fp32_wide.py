@@ -1,6 +1,6 @@
-"""The FP32 passes of 512 lines at both block widths (twice the lines where Ny
-takes whole blocks of them): the step against FP64 at the bar of the FP32 form
-(phi 1e-6 of the FP64 run)."""
+"""The FP32 passes of 512 lines.  The z update of a followed step takes 16 lines
+per block, the x c2r 32 where Ny holds them and 16 otherwise: the step against
+FP64 at the bar of the FP32 form (phi 1e-6 of the FP64 run)."""
 import numpy as np
 import pytest
 
@@ -10,8 +10,9 @@ from helpers import rel_l2
 pytestmark = pytest.mark.gpu
 
 
-# Ny = 16: two blocks of 8 z lines or one of 16; Nx = 512: 16 rows per x block, 32 need Ny >= 32
-@pytest.mark.parametrize("shape", [(64, 32, 512), (32, 64, 512), (512, 16, 32), (512, 32, 64), (512, 32, 512)])
+# Ny = 16: one z block per plane; Nx = 512: 16 rows per x block, 32 need Ny >= 32
+@pytest.mark.parametrize("shape", [(64, 16, 512), (64, 32, 512), (32, 64, 512), (512, 16, 32), (512, 32, 64),
+                                   (512, 32, 512)])
 def test_fp32_steps(shape):
     nx, ny, nz = shape
     phi = P.ic_noisy_constant((nz, ny, nx), 0.45, 0.1, 7)
