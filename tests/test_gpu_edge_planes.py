@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 
 # (Nx, Ny, Nz): one tile of columns to many, every two-level Nz up to 256, both sides of 256 blocks
 SHAPES = [(16, 16, 16), (32, 64, 16), (16, 32, 64), (32, 32, 32), (64, 64, 64), (128, 64, 64), (16, 16, 256),
-          (32, 128, 128), (64, 64, 256), (128, 128, 128)]
+          (32, 128, 128), (64, 64, 256), (128, 128, 128),
+          (64, 32, 512), (32, 16, 512)]   # the planes by kernels of their own; the noise of the bulk through LDS
 
 
 @pytest.mark.parametrize("noise", [P.NOISE_OFF, P.NOISE_DEVICE])

@@ -15,7 +15,7 @@ from oracle import oracle_ctypes as O
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(64, 256, 32), (32, 64, 256), (64, 512, 16), (1024, 32, 16), (128, 64, 64), (256, 16, 128), (512, 32, 32),
-          (32, 512, 32), (64, 64, 128)]   # (Nx, Ny, Nz), all above 2^18 points
+          (32, 512, 32), (64, 64, 128), (32, 32, 512)]   # (Nx, Ny, Nz), all above 2^18 points
 
 
 @pytest.mark.parametrize("shape", SHAPES)
