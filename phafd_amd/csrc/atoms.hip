@@ -830,7 +830,7 @@ __global__ __launch_bounds__(256) void k_ga_pm_rank(int nent, const int *__restr
 // walk was bound by L1 and L2 traffic (a line per 8-byte value); G lanes of
 // one atom share the lines of its x runs.  Thread per atom -> now, us a
 // launch: 161 -> 109 (256^3 FP64, 500k beads, 8 pairs per atom), 6894 -> 2544
-// (512^3 FP32, 2M beads, 87 pairs per atom), 287 -> 104 (512 x 128 x 32 FP64,
+// (512^3 FP32, 2M beads, 87 pairs per atom), 287 -> 86 (512 x 128 x 32 FP64,
 // 63k beads, 87).  What bounds the wide case now: about half the cycles issue
 // arithmetic, and the mu terms' scattered 4-byte stores leave L2 as 45M
 // 64-byte writes, four times the terms' bytes.
@@ -2024,12 +2024,13 @@ static int ilog2(int v) {
 }
 // Lanes per atom of the force walk and the order of its atoms.  16 lanes cover
 // a wide coupling's x runs (5 points at reach 2.75) with fewer cache lines per
-// load, 8 leave fewer lanes idle on a narrow one's few pairs.  Measured, us a
-// launch (8 lanes / 16 lanes / 16 lanes by tiles): 87 pairs per atom, 512^3
-// FP32, 2M beads 3820 / 3067 / 2544 and 512 x 128 x 32 FP64 151 / 131 / 104;
-// 8 pairs per atom, 256^3 FP64, 500k beads 109 / 136 / 139 (8 lanes by tiles:
-// 108, not worth the order's build).  48 pairs per atom (reach 2.25, 128^3):
-// 16 lanes 4% less per step.  24 pairs, three rounds of 8 lanes, is between.
+// load, 8 leave fewer lanes idle on a narrow one's few pairs.  Measured when
+// the walk still read the forces it adds to, us a launch (8 lanes / 16 lanes /
+// 16 lanes by tiles): 87 pairs per atom, 512^3 FP32, 2M beads 3820 / 3067 /
+// 2544 and 512 x 128 x 32 FP64 151 / 131 / 104; 8 pairs per atom, 256^3 FP64,
+// 500k beads 109 / 136 / 139 (8 lanes by tiles: 108, not worth the order's
+// build).  48 pairs per atom (reach 2.25, 128^3): 16 lanes 4% less per step.
+// 24 pairs, three rounds of 8 lanes, is between.
 bool ga_wide(int64_t ng, int64_t nent) { return nent >= 24 * ng; }
 // points per thread of the mu sums: four leave more loads in flight, but a
 // small grid needs its blocks to reach every CU (64^3: 256 blocks of four)

@@ -131,7 +131,7 @@ void launch_ga_density(int ng, const GridView &gv, const GAParams &ga, const dou
 // scanned counts) writes them to ps[].x in ascending grid index, with their
 // atom's q in amq (the am list); launch_ga_pm_count / _place group the am
 // entries by grid point in ascending q (pcnt zeroed by the caller, poff its
-// scan; key, ent scratch): ps[entry].y = its slot in the point's segment.
+// scan; rank, key scratch): ps[entry].y = its slot in the point's segment.
 void launch_ga_am_walk(int ng, const GridView &gv, const double4 *gxb, const int *order, double reachsq, int *cnt,
                        const int *off, int2 *ps, int *amq, hipStream_t s);
 // a wide coupling: many pairs per gathered atom (the force walk's shape)

@@ -163,14 +163,15 @@ struct UpdateParams;
 // fft_r2c_xy: the x and y passes of an r2c.  fft_grad_sep: the gradient of
 // phi by separable spectral derivatives (grids with fft_sep_grad_ok): gx from
 // one x-line kernel, gy and gz from phi's y and z lines and the Nyquist modes
-// of its transform (FP32 and small grids: from the y pass and the z pass); ph
-// receives phihat; gy_k, gz_k are scratch spectra; equal in exact arithmetic
-// to r2c, grad multiply, three c2r / N.  fft_z_update: z pass of mu's r2c, the
-// spectral update of phihat and the z pass of its c2r in one kernel (grids
-// with fft_fused_z_ok); finish with fft_c2r_yx_batch.  origin != nullptr
+// of its transform (FP32, and up to 2^18 points: from the y pass and the z
+// pass); ph receives phihat; gy_k, gz_k are scratch spectra; equal in exact
+// arithmetic to r2c, grad multiply, three c2r / N.  fft_z_update: z pass of
+// mu's r2c, the spectral update of phihat and the z pass of its c2r in one
+// kernel (grids with fft_fused_z_ok); finish with fft_c2r_yx_batch.  origin != nullptr
 // (FP32 form): the k = 0 mode is taken from the FP64 sum there.  store_mu
-// false: muhat of the planes 1 <= kx < Nx/2 is left as the y pass wrote it
-// (for steps whose muhat nobody reads; the update itself is unchanged).
+// false: muhat is left as the y pass wrote it (for steps whose muhat nobody
+// reads; the update itself is unchanged; at Nz = 512 the planes kx = 0 and
+// Nx/2 are written all the same).
 // fft_z_update_next / fft_c2r_next (grids with fft_sep_grad_ok, one
 // system): the update of a step that another step of the run follows, and
 // the c2r of phi together with the next step's gradient: phihat keeps N
