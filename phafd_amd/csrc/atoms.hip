@@ -830,7 +830,7 @@ __global__ __launch_bounds__(256) void k_ga_pm_rank(int nent, const int *__restr
 // walk was bound by L1 and L2 traffic (a line per 8-byte value); G lanes of
 // one atom share the lines of its x runs.  Thread per atom -> now, us a
 // launch: 161 -> 109 (256^3 FP64, 500k beads, 8 pairs per atom), 6894 -> 2544
-// (512^3 FP32, 2M beads, 87 pairs per atom), 287 -> 86 (512 x 128 x 32 FP64,
+// (512^3 FP32, 2M beads, 87 pairs per atom), 287 -> 82 (512 x 128 x 32 FP64,
 // 63k beads, 87).  What bounds the wide case now: about half the cycles issue
 // arithmetic, and the mu terms' scattered 4-byte stores leave L2 as 45M
 // 64-byte writes, four times the terms' bytes.
