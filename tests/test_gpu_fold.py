@@ -28,7 +28,8 @@ def _beads(kind, box, rng):
 
 @pytest.mark.parametrize("zghost", [0, 1])
 @pytest.mark.parametrize("kind,n,box", [("one", 16, 16.0), ("corner", 16, 16.0), ("edges", 32, 32.0),
-                                        ("inside", 16, 16.0), ("all", 32, 32.0), ("all", 16, 8.0), ("corner", 8, 6.0)])
+                                        ("inside", 16, 16.0), ("all", 32, 32.0), ("all", 16, 8.0), ("corner", 8, 6.0),
+                                        ("corner", 8, 4.0), ("all", 16, 4.0)])   # the last two: swaps that share atoms
 def test_forces_of_folded_images(kind, n, box, zghost):
     rng = np.random.default_rng(n)
     xyz = _beads(kind, box, rng)
